@@ -1606,12 +1606,18 @@ inline uint64_t mla_max_workers(bool sparse, int rows, int topk, int n_sinks) {
   const uint64_t need = (uint64_t(rows) * per_row + kMlaSparseShare - 1) / kMlaSparseShare;
   return need > grid ? need : grid;
 }
+// Partial slots: at most two per worker for rows whose keys span several
+// shares. With sinks every row writes partials (one for the sinks, one per
+// share its keys touch): a share's rows inside it add one each, so two per row
+// on top of the shares' boundaries.
+inline uint64_t mla_slots(uint64_t workers, int rows, int n_sinks) {
+  return 2 * workers + (n_sinks > 0 ? 2 * uint64_t(rows) : 0);
+}
 // Workspace: plan words | row_pos | row_seq | row_slot | start_row | partial
-// O | partial (m, l). Partial slots: one per row for the sinks, and at most
-// two per worker for the key shares.
+// O | partial (m, l).
 inline uint64_t mla_workspace(int rows, int heads, bool sparse, int topk, int n_sinks) {
   const uint64_t workers = mla_max_workers(sparse, rows, topk, n_sinks);
-  const uint64_t slots = 2 * workers + (n_sinks > 0 ? uint64_t(rows) : 0);
+  const uint64_t slots = mla_slots(workers, rows, n_sinks);
   return kQueueBytes + 2 * align16(uint64_t(rows) * 8) + align16(uint64_t(rows) * 4) +
          align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 2 * sizeof(float));
 }
@@ -1693,7 +1699,7 @@ int32_t mla_run(const MlaCall &c, const char *what) {
   p.self_plan = c.num_rows <= kMlaSelfPlanRows &&
                 int64_t(c.num_rows) * (int64_t(c.max_context) + p.row_cost + p.sink_units + kMlaTile) <
                     (int64_t(1) << 31) &&
-                2 * max_workers + uint64_t(c.num_rows) < 0xFFFFu;
+                mla_slots(max_workers, c.num_rows, 1) < 0xFFFFu;
   uint8_t *ws = static_cast<uint8_t *>(c.workspace);
   p.plan = reinterpret_cast<int32_t *>(ws);
   ws += kQueueBytes;
@@ -1705,7 +1711,7 @@ int32_t mla_run(const MlaCall &c, const char *what) {
   ws += align16(uint64_t(c.num_rows) * 8);
   p.start_row = reinterpret_cast<int32_t *>(ws);
   ws += align16(max_workers * 4);
-  const uint64_t slots = 2 * max_workers + (c.n_sinks > 0 ? uint64_t(c.num_rows) : 0);
+  const uint64_t slots = mla_slots(max_workers, c.num_rows, c.n_sinks);
   p.part_o = reinterpret_cast<uint16_t *>(ws);
   p.part_ml = reinterpret_cast<float *>(p.part_o + slots * c.heads * 512);
   hipStream_t s = static_cast<hipStream_t>(c.stream);
