@@ -1,0 +1,709 @@
+// Packed-MLA window attention of prompt chunks (gfx950, bf16 latent rows).
+//
+// The operation of ifattn_mla_window_attention_bf16 (see mla_decode.hip for the
+// row and window rules) for calls whose sequences have several query rows. The
+// rows of a chunk see almost the same keys, so a workgroup takes 128 (query
+// row, head) columns at once and every staged key tile is scored against all of
+// them; the row-by-row kernel stages the same tile again for every row and
+// fills 16 of the MFMA columns with one row's heads (fewer heads leave the
+// rest empty; here six heads pack 21 rows into 126 columns).
+//
+// Bound: MFMA and LDS operand reads. A 32-key tile against 128 columns is 8.9
+// MFLOP (0.9 us of one CU's bf16 rate) and 400 KB of LDS reads, for 36 KB moved
+// from L2; it takes 2.2-2.4 us (2.2 without the loads). A group's start (q and
+// the first tile) takes 6 us and its partial output 6 us. Measured against the
+// row-by-row kernel: 756 rows x 16 heads in three chunks, window 2048, 128
+// sinks 269 -> 105 us a call with the writer; 2048 rows over 8192 earlier keys
+// 688 us (954 TFLOP/s).
+//
+// Layout: eight waves, two per SIMD. Scores are split by columns: wave w owns
+// columns [16w, 16w + 16) with q in registers (72 VGPRs), reads the whole tile
+// as the A operand, and keeps its columns' running max and sum, so the softmax
+// needs no exchange. PV is split by dims: wave w owns latent dims [64w, 64w +
+// 64) of all 128 columns (128 accumulators), with the transposed V operand
+// (ds_read_b64_tr_b16) read once per tile by one wave only; the
+// probabilities travel through LDS (8 KB per tile) in MFMA operand layout.
+// Splitting PV by columns instead would read the tile's V bytes eight times and
+// needs 128 accumulators as well.
+//
+// Pipeline: one barrier per tile. Iteration i waits for tile i, issues tile
+// i + 1 into the third ring slot, runs PV of tile i - 1 and scores of tile i.
+// Running-max updates travel with the probabilities: a wave whose columns grew
+// by more than 2^8 publishes the rescale factors next to P and PV applies them.
+//
+// Sinks are key tiles in front of the row's own: their keys and values differ,
+// so a sink tile takes two ring slots (keys: scores only; values: PV only).
+//
+// Work split: groups of floor(128 / heads) rows of one sequence, weighted by
+// their tiles plus a start cost, cut into equal contiguous shares, one per
+// persistent workgroup (the scheme of mla_decode.hip); a group over several
+// shares leaves one partial per share for the merge launch. A worker's share
+// holds at most two split pieces, one continuing a group of an earlier worker
+// (slot 2v) and one starting a group that a later worker ends (slot 2v + 1), so
+// slots need no plan. Partials are O / l as fp16 under a power-of-two scale per
+// (column, 64 dims): half the bytes of fp32 and 2^-11 of the largest value at
+// worst, below the rounding of the bf16 probabilities.
+#include "common.h"
+#include "ifattn_internal.h"
+#include "mla_chunk.h"
+#include "split_k.h"
+
+namespace ifattn {
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kThreads = 64 * kWaves;
+constexpr int kCols = 16 * kWaves;
+constexpr int kTile = 32;
+constexpr uint32_t kRow = 1152;                 // bytes of a latent row
+constexpr uint32_t kSlot = kTile * kRow;        // one staged tile: latent rows, then
+constexpr uint32_t kRope = kTile * 1024;        // the rope rows from this byte on
+constexpr int kStages = 3;
+#ifndef IFATTN_CHUNK_AHEAD
+#define IFATTN_CHUNK_AHEAD 1
+#endif
+constexpr int kAhead = IFATTN_CHUNK_AHEAD;  // LDS operands in flight ahead of the MFMAs
+constexpr int kStart = 3;      // work units (tiles) charged per group: q loads and output stores
+constexpr int kMinShare = 8;   // smallest share, in tiles
+constexpr int kLdsGroups = kThreads;  // calls of at most this many groups and sequences plan in LDS
+
+struct ChunkParams {
+  const uint16_t *q;            // [rows, heads, 576]
+  const uint8_t *cache;         // rows of 1152 bytes
+  const int32_t *block_tables, *kv_lens, *cu_q;
+  const uint16_t *sink_k, *sink_v;
+  uint16_t *out;                // [rows, heads, 512]
+  int32_t *head;                // [2] groups, total units
+  int32_t *gpre;                // [seqs] groups of earlier sequences
+  int32_t *gseq;                // [groups] sequence of each group
+  int32_t *gpos;                // [groups + 1] first work unit of each group
+  uint16_t *part_o;             // [2 * grid, 128, 512] fp16
+  float *part_sc;               // [2 * grid, 128, 8]
+  float2 *part_ml;              // [2 * grid, 128]
+  int64_t num_blocks;
+  int num_seqs, num_rows, heads, rows_per, table_stride, block_size, max_context, window, n_sinks;
+  int sink_tiles, groups_max, grid, lds_plan;
+  float scale_log2;
+};
+
+// Keys of one group: rows [first, first + rows) of sequence `seq`; row t sees
+// positions [lo(t), hi(t)).
+struct Group {
+  int seq, row0, rows;  // row0: packed row of the group's first row
+  int c0;               // causal keys of the group's first row (unclamped)
+  int lo, hi, base, tiles;
+};
+__device__ __forceinline__ int clamp_keys(const ChunkParams &p, int causal) {
+  return causal < 0 ? 0 : (causal > p.max_context ? p.max_context : causal);
+}
+__device__ __forceinline__ int window_lo(const ChunkParams &p, int causal) {
+  return p.window > 0 && causal > p.window ? causal - p.window : 0;
+}
+__device__ __forceinline__ int seq_rows(const ChunkParams &p, int seq, int &start) {
+  start = ld_const(p.cu_q + seq);
+  const int end = ld_const(p.cu_q + seq + 1);
+  return (end < p.num_rows ? end : p.num_rows) - start;
+}
+__device__ __forceinline__ Group group_of(const ChunkParams &p, int seq, int index) {
+  Group g;
+  int start;
+  const int count = seq_rows(p, seq, start);
+  const int first = index * p.rows_per;
+  int kv = ld_const(p.kv_lens + seq);
+  kv = kv > p.max_context ? p.max_context : kv;
+  g.seq = seq;
+  g.row0 = start + first;
+  g.rows = count - first < p.rows_per ? count - first : p.rows_per;
+  g.c0 = kv - count + first + 1;
+  g.lo = window_lo(p, clamp_keys(p, g.c0));
+  g.hi = clamp_keys(p, g.c0 + g.rows - 1);
+  g.base = g.lo & ~(kTile - 1);
+  // A group without keys keeps one (empty) tile: its rows are written too.
+  g.tiles = g.hi > g.base ? (g.hi - g.base + kTile - 1) / kTile : 1;
+  return g;
+}
+// Largest s with pre[s] <= g.
+__device__ __forceinline__ int seq_of_group(const int32_t *pre, int num_seqs, int g) {
+  int a = 0, b = num_seqs - 1;
+  while (a < b) {
+    const int m = (a + b + 1) >> 1;
+    if (pre[m] <= g) a = m; else b = m - 1;
+  }
+  return a;
+}
+
+// Inclusive scan over NT threads; *total gets the workgroup's sum.
+template <int NT>
+__device__ __forceinline__ int scan_sum(int x, int *wt, int *total) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int y = __shfl_up(x, off, 64);
+    if (lane >= off) x += y;
+  }
+  if (lane == 63) wt[wv] = x;
+  __syncthreads();
+  int before = 0, all = 0;
+#pragma unroll
+  for (int u = 0; u < NT / 64; ++u) {
+    const int t = wt[u];
+    before += u < wv ? t : 0;
+    all += t;
+  }
+  __syncthreads();  // wt is reused by the next scan
+  *total = all;
+  return before + x;
+}
+
+// The plan, by one workgroup of NT threads, into pre / seq / pos (LDS in the
+// attention workgroups of small calls, the workspace in the plan launch).
+template <int NT>
+__device__ __forceinline__ void make_plan(const ChunkParams &p, int32_t *pre, int32_t *gseq,
+                                          int32_t *pos, int *wt, int &groups, int &total) {
+  const int tid = threadIdx.x;
+  int carry = 0;
+  for (int b = 0; b < p.num_seqs; b += NT) {
+    const int s = b + tid;
+    int n = 0;
+    if (s < p.num_seqs) {
+      int start;
+      const int count = seq_rows(p, s, start);
+      n = count > 0 ? (count + p.rows_per - 1) / p.rows_per : 0;
+    }
+    int all;
+    const int incl = scan_sum<NT>(n, wt, &all);
+    if (s < p.num_seqs) pre[s] = carry + incl - n;
+    carry += all;
+  }
+  groups = carry < p.groups_max ? carry : p.groups_max;
+  __syncthreads();
+  carry = 0;
+  for (int b = 0; b < groups; b += NT) {
+    const int g = b + tid;
+    int w = 0, s = 0;
+    if (g < groups) {
+      s = seq_of_group(pre, p.num_seqs, g);
+      w = kStart + p.sink_tiles + group_of(p, s, g - pre[s]).tiles;
+    }
+    int all;
+    const int incl = scan_sum<NT>(w, wt, &all);
+    if (g < groups) {
+      gseq[g] = s;
+      pos[g] = carry + incl - w;
+    }
+    carry += all;
+  }
+  total = carry;
+  if (tid == 0) pos[groups] = total;
+  __syncthreads();
+}
+__device__ __forceinline__ int share_units(const ChunkParams &p, int total, int &workers) {
+  workers = total / kMinShare < p.grid ? total / kMinShare : p.grid;
+  workers = workers < 1 ? 1 : workers;
+  return (total + workers - 1) / workers;
+}
+// A share ends at v * share, or at a group's end when one lies within `snap`
+// units: a split costs its group a second start, two partials and their merge.
+__device__ __forceinline__ int share_snap(int share) { return kStart + share / 16; }
+// Interior share ends of the group [a, b): workers first .. last start inside it.
+__device__ __forceinline__ void group_splits(int a, int b, int share, int &first, int &last) {
+  const int snap = share_snap(share);
+  first = (a + snap) / share + 1;
+  last = (b - snap + share - 1) / share - 1;  // largest v with v * share < b - snap
+}
+
+__global__ __launch_bounds__(1024) void mla_chunk_plan_kernel(ChunkParams p) {
+  __shared__ int wt[16];
+  int groups, total;
+  make_plan<1024>(p, p.gpre, p.gseq, p.gpos, wt, groups, total);
+  if (threadIdx.x == 0) {
+    p.head[0] = groups;
+    p.head[1] = total;
+  }
+}
+
+// Bits of row & 15 as chunk bits (0, 3, 1, 2).
+__device__ __forceinline__ int latent_key(int row) {
+  return (row & 1) | ((row & 2) << 2) | ((row & 12) >> 1);
+}
+__device__ __forceinline__ int rope_key(int row) { return (row >> 1) & 7; }
+__device__ __forceinline__ int tile_token(int g, int j) { return j < 4 ? 4 * g + j : 12 + 4 * g + j; }
+
+// The lane index, computed anew: the accumulators and q leave no registers to
+// keep per-lane addresses across the tile loop, and a spilled one is reloaded
+// behind the tile loads in flight.
+__device__ __forceinline__ int fresh_lane() {
+  int x;
+  asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(x));
+  return x;
+}
+
+__global__ __launch_bounds__(kThreads) void mla_chunk_kernel(ChunkParams p) {
+  __shared__ __align__(16) uint8_t ring[kStages * kSlot];
+  __shared__ __align__(16) u32x4 s_p[2][kWaves][64];  // probabilities, B operand layout
+  __shared__ float s_alpha[2][kCols];
+  __shared__ int s_flag[2][kWaves], s_end[2], s_first;
+  __shared__ float2 s_ml[kCols];
+  __shared__ int s_pre[kLdsGroups], s_seq[kLdsGroups], s_pos[kLdsGroups + 1], s_wt[kWaves];
+
+  const int tid = threadIdx.x, lane = tid & 63, w = uniform(int(tid >> 6));
+  const int c = lane & 15, g4 = lane >> 4;
+  int groups, total;
+  const int32_t *pre = p.gpre, *gseq = p.gseq, *pos = p.gpos;
+  if (p.lds_plan) {
+    make_plan<kThreads>(p, s_pre, s_seq, s_pos, s_wt, groups, total);
+    pre = s_pre;
+    gseq = s_seq;
+    pos = s_pos;
+    if (blockIdx.x == 0) {  // for the merge
+      if (tid < p.num_seqs) p.gpre[tid] = s_pre[tid];
+      if (tid < groups) p.gseq[tid] = s_seq[tid];
+      if (tid < groups) p.gpos[tid] = s_pos[tid];
+      if (tid == 0) {
+        p.gpos[groups] = total;
+        p.head[0] = groups;
+        p.head[1] = total;
+      }
+    }
+  } else {
+    groups = ld_const(p.head);
+    total = ld_const(p.head + 1);
+  }
+  groups = uniform(groups);
+  total = uniform(total);
+  int workers;
+  const int share = uniform(share_units(p, total, workers));
+  // Consecutive shares (whose rows see the same keys) run on one XCD.
+  const int per_xcd = (workers + 7) / 8;
+  const int slice = int(blockIdx.x) >> 3;
+  const int v = (int(blockIdx.x) & 7) * per_xcd + slice;
+  if (slice >= per_xcd || v >= workers) return;
+  // The share's ends and its first group: every thread tests its groups.
+  const int snap = share_snap(share);
+  if (tid < 2) s_end[tid] = total;
+  if (tid == 2) s_first = groups;
+  __syncthreads();
+  for (int g = tid; g < groups; g += kThreads) {
+    const int a = pos[g], b = pos[g + 1];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const int raw = (v + e) * share;
+      if (raw < a || raw >= b) continue;
+      const bool down = raw - a <= snap, up = !down && b - raw <= snap;
+      s_end[e] = down ? a : (up ? b : raw);
+      if (e == 0) s_first = up ? g + 1 : g;
+    }
+  }
+  __syncthreads();
+  const int u0 = uniform(s_end[0]), u1 = uniform(s_end[1]);
+  int gi = uniform(s_first);
+
+  const uint32_t ring_base = lds_addr(ring);
+  const int bs = p.block_size, bs_log2 = __builtin_ctz(uint32_t(p.block_size));
+  for (; gi < groups; ++gi) {
+    const int gp = uniform(pos[gi]);
+    if (gp >= u1) break;
+    const int seq = uniform(gseq[gi]);
+    Group gr = group_of(p, seq, gi - uniform(pre[seq]));
+    const int all_tiles = p.sink_tiles + gr.tiles;
+    const int first = gp + kStart;
+    int j0 = u0 - first, j1 = u1 - first;
+    j0 = j0 < 0 ? 0 : j0;
+    j1 = j1 < all_tiles ? j1 : all_tiles;
+    if (j0 >= j1) continue;
+    j0 = uniform(j0);
+    j1 = uniform(j1);
+    const int ncols = gr.rows * p.heads;
+    const int nb_live = (ncols + 15) / 16;
+    const bool mine = w < nb_live;  // this wave has columns
+
+    // This lane's column and its key range.
+    const int col = 16 * w + c;
+    const int colc = col < ncols ? col : ncols - 1;
+    const int causal = clamp_keys(p, gr.c0 + colc / p.heads);
+    const int col_lo = window_lo(p, causal), col_hi = causal;
+    const int lo_max = window_lo(p, gr.hi);               // start of the last row's window
+    const int hi_min = clamp_keys(p, gr.c0);              // end of the first row's
+    // Loads of this piece: two per sink tile (keys, values), one per key tile.
+    const int nsk = uniform(j0 < p.sink_tiles ? (j1 < p.sink_tiles ? j1 : p.sink_tiles) - j0 : 0);
+    const int kt0 = j0 > p.sink_tiles ? j0 - p.sink_tiles : 0;  // first key tile
+    const int nkt = j1 > p.sink_tiles ? j1 - p.sink_tiles - kt0 : 0;
+    const int nload = 2 * nsk + nkt;
+    // Block ids of a 64-block window, one per lane (entries past the keys read 0).
+    const int nblk = gr.hi > 0 ? (gr.hi - 1) / bs + 1 : 0;
+    int wblk0 = (gr.base + kt0 * kTile) >> bs_log2, lane_blocks = 0;
+    const auto rw = make_rsrc(p.block_tables + int64_t(seq) * p.table_stride, uint32_t(nblk) * 4);
+    auto load_window = [&]() {
+      const int b = int(buf_load_x1(rw, uint32_t(wblk0 + lane) * 4));
+      lane_blocks = b < 0 ? 0 : (b >= p.num_blocks ? int(p.num_blocks - 1) : b);
+    };
+    load_window();
+    // A staged tile is 32 latent rows of 1024 bytes, then 32 rope rows of 128;
+    // the 16-byte chunks of a row are XOR-swizzled so that K operand reads (16
+    // rows, one chunk) and transposing V reads (4 rows, every other chunk of
+    // eight) touch distinct banks. Rows r and r + 16 share a key. Load k < 4 of
+    // wave w moves latent row 8k + w, load 4 of waves 0-3 rope rows 8w .. 8w + 7.
+    auto issue = [&](int i, int slot) {
+      const uint32_t dst = ring_base + uint32_t(slot) * kSlot;
+      const int ln = fresh_lane();
+      const uint32_t src_l = 16u * uint32_t(ln ^ latent_key(w));  // row 8k + w: key bit 2 = k & 1
+      const uint32_t src_r = 1024u + uint32_t(ln >> 3) * kRow +
+                             16u * uint32_t((ln & 7) ^ rope_key(8 * w + (ln >> 3)));
+      // Rows [r0, r1) of the tile live in `rs`, whose base is tile row `at`;
+      // offsets of earlier rows wrap past the extent and land as zeros, like
+      // rows past the end.
+      auto move = [&](u32x4 rs, uint32_t pitch, int at, bool upper_half) {
+        const int k0 = upper_half ? 2 : 0;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          lds_dma16(rs, (src_l ^ (64u * uint32_t(k))) + uint32_t(8 * (k0 + k) + w - at) * pitch,
+                    dst + uint32_t(8 * (k0 + k) + w) * 1024u);
+        if (pitch == kRow && w < 4 && (w < 2) != upper_half)
+          lds_dma16(rs, src_r + uint32_t(8 * w - at) * pitch, dst + kRope + uint32_t(w) * 1024u);
+      };
+      if (i < 2 * nsk) {
+        const int s = j0 + (i >> 1);
+        const int n = p.n_sinks - s * kTile < kTile ? p.n_sinks - s * kTile : kTile;
+        const bool is_v = i & 1;
+        const uint32_t pitch = is_v ? 1024u : kRow;
+        const u32x4 rs = raw_rsrc((is_v ? p.sink_v : p.sink_k) + int64_t(s) * kTile * (pitch / 2),
+                                  uint32_t(n) * pitch);
+        move(rs, pitch, 0, false);
+        move(rs, pitch, 0, true);
+        return;
+      }
+      const int t0 = gr.base + (kt0 + i - 2 * nsk) * kTile;
+      const int lower = gr.lo > t0 ? gr.lo - t0 : 0;
+      const int upper = gr.hi - t0 < kTile ? gr.hi - t0 : kTile;
+      if (((t0 + kTile - 1) >> bs_log2) - wblk0 >= 64) {
+        wblk0 = t0 >> bs_log2;
+        load_window();
+      }
+      // One block, or two 16-row blocks.
+      auto part = [&](int r0, int r1, int blk_at) {
+        const int a = lower > r0 ? lower : r0, b = upper < r1 ? upper : r1;
+        const int blk = __builtin_amdgcn_readlane(lane_blocks, blk_at);
+        const int64_t tok = int64_t(blk) * bs + (t0 & (bs - 1)) + (a - r0);
+        return raw_rsrc(p.cache + tok * kRow, b > a ? uint32_t(b - a) * kRow : 0u);
+      };
+      const int at = (t0 >> bs_log2) - wblk0;
+      if (bs >= kTile) {
+        const u32x4 rs = part(0, kTile, at);
+        move(rs, kRow, lower, false);
+        move(rs, kRow, lower, true);
+      } else {
+        move(part(0, 16, at), kRow, lower, false);
+        move(part(16, 32, at + 1), kRow, lower > 16 ? lower : 16, true);
+      }
+    };
+
+    issue(0, 0);
+    u32x4 qv[18];
+    {
+      const auto rq = make_rsrc(p.q + int64_t(gr.row0) * p.heads * 576, uint32_t(ncols) * 1152u);
+#pragma unroll
+      for (int s = 0; s < 18; ++s)  // columns past the group read as zeros
+        qv[s] = buf_load_x4(rq, uint32_t(col) * 1152u + uint32_t(32 * s + 8 * g4) * 2u);
+    }
+
+    f32x4 oacc[8][4];
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) oacc[nb][b] = f32x4{0, 0, 0, 0};
+    float m_run = -INFINITY, l_run = 0.0f;
+
+    auto pv = [&](int slot, int buf) {
+      const uint32_t grown = uint32_t(__ballot(s_flag[buf][fresh_lane() & 7] != 0)) & 0xFFu;
+      if (grown) {
+#pragma unroll
+        for (int nb = 0; nb < 8; ++nb)
+          if ((grown >> nb) & 1u) {
+            const float a = s_alpha[buf][16 * nb + (fresh_lane() & 15)];
+#pragma unroll
+            for (int b = 0; b < 4; ++b) oacc[nb][b] *= a;
+          }
+      }
+      // V operand of block b: MFMA row m is dim 64w + 16(m >> 2) + 4b + (m & 3),
+      // so a lane ends with 16 consecutive dims of its column. Rows
+      // tile_token(g, c >> 2) (+ 16), dims 64w + 16(c & 3) + 4b: the blocks are
+      // one address under a xor.
+      const int ln = fresh_lane(), lc = ln & 15, vrow = 4 * (ln >> 4) + (lc >> 2);
+      const uint32_t va0 =
+          uint32_t(vrow) * 1024u + 16u * uint32_t((8 * w + 2 * (lc & 3)) ^ latent_key(vrow));
+      const __attribute__((address_space(3))) char *vt =
+          (const __attribute__((address_space(3))) char *)(ring) + slot * int(kSlot);
+      typedef short s16x4 __attribute__((ext_vector_type(4)));
+      typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+      u32x4 a[4];
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vt + (va0 ^ (8u * b))));
+        const s16x4 hi =
+            __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(vt + (va0 ^ (8u * b)) + 16 * 1024));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+        a[b] = u32x4{l2[0], l2[1], h2[0], h2[1]};
+      }
+      // The next column blocks' probabilities are in flight while one is used
+      // (blocks without columns multiply what lies there; nothing reads them).
+      u32x4 pb[kAhead + 1];
+#pragma unroll
+      for (int n = 0; n < kAhead; ++n) pb[n] = s_p[buf][n][ln];
+#pragma unroll
+      for (int n = 0; n < 8; ++n) {
+        if (n + kAhead < 8) pb[(n + kAhead) % (kAhead + 1)] = s_p[buf][n + kAhead][ln];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) oacc[n][b] = mfma16x16x32(a[b], pb[n % (kAhead + 1)], oacc[n][b]);
+      }
+    };
+    // Scores and online softmax of the tile in `slot`: key r of the tile is
+    // visible to this lane's column when lo <= r < hi.
+    auto scores = [&](int slot, int buf, int lo, int hi, bool masked) {
+      if (!mine) return;
+      // K operand: key c (+ 16), dims 32s + 8g (chunk 4s + g): steps s < 4 are
+      // one address under a xor, s + 4 an immediate away.
+      const uint8_t *kt = ring + slot * int(kSlot);
+      const int ln = fresh_lane(), lc = ln & 15, lg = ln >> 4;
+      const uint32_t ka0 = uint32_t(lc) * 1024u + 16u * uint32_t(lg ^ latent_key(lc));
+      const uint32_t kr0 = kRope + uint32_t(lc) * 128u + 16u * uint32_t(lg ^ rope_key(lc));
+      f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
+      // The next k-steps' operands are in flight while one is used.
+      u32x4 kb[kAhead + 1][2];
+      auto load = [&](int s) {
+        const uint8_t *k = kt + ((s < 16 ? ka0 : kr0) ^ (64u * uint32_t(s & 3))) + (s < 16 ? 256 * (s >> 2) : 0);
+        kb[s % (kAhead + 1)][0] = load_u32x4(k);
+        kb[s % (kAhead + 1)][1] = load_u32x4(k + (s < 16 ? 16 * 1024 : 16 * 128));
+      };
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) load(s);
+#pragma unroll
+      for (int s = 0; s < 18; ++s) {
+        if (s + kAhead < 18) load(s + kAhead);
+        __builtin_amdgcn_sched_barrier(0);
+        s0 = mfma16x16x32(kb[s % (kAhead + 1)][0], qv[s], s0);
+        s1 = mfma16x16x32(kb[s % (kAhead + 1)][1], qv[s], s1);
+      }
+      float x[8];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[r] = s0[r] * p.scale_log2;
+        x[4 + r] = s1[r] * p.scale_log2;
+      }
+      if (masked) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const int t = tile_token(lg, j);
+          x[j] = t >= lo && t < hi ? x[j] : -INFINITY;
+        }
+      }
+      float tmax = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])),
+                         fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+      tmax = max_xor32(max_xor16(tmax));
+      const bool grow = __any(tmax > m_run + 8.0f);
+      if (grow) {
+        const float m_new = fmaxf(m_run, tmax);
+        const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
+        if (lg == 0) s_alpha[buf][16 * w + lc] = alpha;
+      }
+      if (ln == 0) s_flag[buf][w] = grow ? 1 : 0;
+      const float m_use = m_run == -INFINITY ? 0.0f : m_run;
+      float pr[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) pr[j] = fast_exp2(x[j] - m_use);
+      l_run += ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
+      s_p[buf][w][ln] = u32x4{pack_bf16x2(pr[0], pr[1]), pack_bf16x2(pr[2], pr[3]),
+                                pack_bf16x2(pr[4], pr[5]), pack_bf16x2(pr[6], pr[7])};
+    };
+    if (!mine && lane < 2) s_flag[lane][w] = 0;
+
+    // Interval i (after the barrier that publishes tile i): the PV due in it,
+    // then the scores of tile i.
+    int cur = 0, prev = 2;  // ring slots of tiles i and i - 1
+    for (int i = 0; i < nload; ++i) {
+      const int next = cur == 2 ? 0 : cur + 1;
+      const bool sink = i < 2 * nsk;
+      const bool sink_v = sink && (i & 1);
+      lds_dma_wait<0>();  // tile i (tile i + 1 is issued below)
+      __syncthreads();
+      if (i + 1 < nload) issue(i + 1, next);
+      if (sink ? sink_v : i > 2 * nsk) pv(sink ? cur : prev, (i + 1) & 1);
+      if (!sink_v) {
+        const int t0 = sink ? (j0 + (i >> 1)) * kTile : gr.base + (kt0 + i - 2 * nsk) * kTile;
+        scores(cur, i & 1, (sink ? 0 : col_lo) - t0, (sink ? p.n_sinks : col_hi) - t0,
+               sink ? t0 + kTile > p.n_sinks : (t0 < lo_max || t0 + kTile > hi_min));
+      }
+      prev = cur;
+      cur = next;
+    }
+    if (mine) {
+      const float l_tot = sum_xor32(sum_xor16(l_run));
+      if (g4 == 0) s_ml[col] = make_float2(m_run, l_tot);
+    }
+    __syncthreads();
+    if (nkt > 0) pv(prev, (nload - 1) & 1);  // the last key tile
+
+    const bool whole = j0 == 0 && j1 == all_tiles;
+    const int slot = 2 * v + (j0 > 0 ? 0 : 1);
+#pragma unroll
+    for (int nb = 0; nb < 8; ++nb) {
+      const int oc = 16 * nb + c;
+      if (nb >= nb_live) break;
+      const float2 ml = s_ml[oc];
+      const float inv = ml.y > 0.0f ? 1.0f / ml.y : 0.0f;
+      const int d0 = 64 * w + 16 * g4;
+      if (whole) {
+        if (oc < ncols) {
+          uint16_t *op = p.out + (int64_t(gr.row0) * p.heads + oc) * 512 + d0;
+#pragma unroll
+          for (int b = 0; b < 4; b += 2) {
+            const f32x4 x = oacc[nb][b] * inv, y = oacc[nb][b + 1] * inv;
+            store_u32x4(op + 4 * b, u32x4{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]),
+                                          pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3])});
+          }
+        }
+        continue;
+      }
+      float amax = 0.0f;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        oacc[nb][b] *= inv;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) amax = fmaxf(amax, fabsf(oacc[nb][b][r]));
+      }
+      amax = max_xor32(max_xor16(amax));
+      const float qs = f16_range_scale(amax);
+      const int64_t prow = int64_t(slot) * kCols + oc;
+      uint16_t *po = p.part_o + prow * 512 + d0;
+      auto half2 = [&](float a, float b) {
+        const f16x2 h = {_Float16(a * qs), _Float16(b * qs)};
+        return __builtin_bit_cast(uint32_t, h);
+      };
+#pragma unroll
+      for (int b = 0; b < 4; b += 2) {
+        const f32x4 x = oacc[nb][b], y = oacc[nb][b + 1];
+        store_u32x4(po + 4 * b, u32x4{half2(x[0], x[1]), half2(x[2], x[3]), half2(y[0], y[1]),
+                                      half2(y[2], y[3])});
+      }
+      if (g4 == 0) p.part_sc[prow * 8 + w] = 1.0f / qs;
+      if (w == 0 && g4 == 0) p.part_ml[prow] = ml;
+    }
+    __syncthreads();  // the ring, P and (m, l) are reused by the next group
+  }
+}
+
+// Combine the partials of one group: one column per wave, four per workgroup;
+// lane l owns dims 8l .. 8l + 7.
+__global__ __launch_bounds__(256) void mla_chunk_merge_kernel(ChunkParams p) {
+  const int g = blockIdx.x;
+  if (g >= ld_const(p.head)) return;
+  int workers;
+  const int share = share_units(p, ld_const(p.head + 1), workers);
+  int va, vb;
+  group_splits(ld_const(p.gpos + g), ld_const(p.gpos + g + 1), share, va, vb);
+  if (va > vb) return;  // one piece: written by the attention kernel
+  const int seq = ld_const(p.gseq + g);
+  const Group gr = group_of(p, seq, g - ld_const(p.gpre + seq));
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = vb - va + 2;
+  auto row_of = [&](int k, int col) {
+    return int64_t(k == 0 ? 2 * va - 1 : 2 * (va + k - 1)) * kCols + col;
+  };
+  const int col = blockIdx.y * 4 + wave;
+  if (col >= gr.rows * p.heads) return;
+  float mx = -INFINITY;
+  for (int k = lane; k < n; k += 64) mx = fmaxf(mx, p.part_ml[row_of(k, col)].x);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) mx = wave_max_xor(mx, m);
+  float l = 0.0f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll 4
+  for (int k = 0; k < n; ++k) {
+    const int64_t r = row_of(k, col);
+    const float2 ml = p.part_ml[r];
+    const u32x4 h = load_u32x4(p.part_o + r * 512 + 8 * lane);
+    const float sc = p.part_sc[r * 8 + (lane >> 3)];
+    const float wk = ml.y > 0.0f ? fast_exp2(ml.x - mx) * ml.y : 0.0f;
+    l += wk;
+    const float f = wk * sc;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const uint32_t word = h[e];  // (a bit cast of the element itself reads element 0)
+      const f16x2 x = __builtin_bit_cast(f16x2, word);
+      acc[2 * e] += f * float(x[0]);
+      acc[2 * e + 1] += f * float(x[1]);
+    }
+  }
+  const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+  store_u32x4(p.out + (int64_t(gr.row0) * p.heads + col) * 512 + 8 * lane,
+              u32x4{pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv),
+                    pack_bf16x2(acc[4] * inv, acc[5] * inv), pack_bf16x2(acc[6] * inv, acc[7] * inv)});
+}
+
+}  // namespace
+
+// Workspace: head | groups of earlier sequences | sequence and first unit of
+// each group | partials. A call has at most num_rows groups and sequences.
+uint64_t mla_chunk_workspace(int32_t num_rows) {
+  if (num_rows < 2) return 0;
+  const uint64_t rows = uint64_t(num_rows), slots = 2 * uint64_t(device_cus());
+  return 16 + 2 * align16(4 * rows) + align16(4 * rows + 4) +
+         slots * kCols * (512 * sizeof(uint16_t) + 8 * sizeof(float) + sizeof(float2));
+}
+
+bool mla_chunk_takes(const MlaChunkCall &c) {
+  // Two rows per sequence on average: below that most rows are single decode
+  // rows, which the row kernel streams at HBM rate.
+  if (!c.cu_q || int64_t(c.num_rows) < 2 * int64_t(c.num_seqs)) return false;
+  if (c.n_sinks > 0 && (!aligned16(c.sink_k) || !aligned16(c.sink_v))) return false;
+  if (c.workspace_bytes < mla_chunk_workspace(c.num_rows)) return false;
+  const int64_t groups = int64_t(c.num_rows) / (kCols / c.heads) + c.num_seqs;
+  return groups * (kStart + (int64_t(c.n_sinks) + c.max_context) / kTile + 2) < (int64_t(1) << 31);
+}
+
+void launch_mla_chunk(const MlaChunkCall &c) {
+  ChunkParams p{};
+  p.q = static_cast<const uint16_t *>(c.q);
+  p.cache = static_cast<const uint8_t *>(c.cache);
+  p.block_tables = c.block_tables;
+  p.kv_lens = c.kv_lens;
+  p.cu_q = c.cu_q;
+  p.sink_k = static_cast<const uint16_t *>(c.sink_k);
+  p.sink_v = static_cast<const uint16_t *>(c.sink_v);
+  p.out = static_cast<uint16_t *>(c.out);
+  p.num_blocks = c.num_blocks;
+  p.num_seqs = c.num_seqs;
+  p.num_rows = c.num_rows;
+  p.heads = c.heads;
+  p.rows_per = kCols / c.heads;
+  p.table_stride = c.table_stride;
+  p.block_size = c.block_size;
+  p.max_context = c.max_context;
+  p.window = c.window;
+  p.n_sinks = c.n_sinks;
+  p.sink_tiles = (c.n_sinks + kTile - 1) / kTile;
+  p.groups_max = c.num_rows / p.rows_per + c.num_seqs;
+  p.grid = device_cus();
+  p.lds_plan = p.groups_max <= kLdsGroups && c.num_seqs <= kLdsGroups;
+  p.scale_log2 = c.scale * kLog2e;
+  uint8_t *ws = static_cast<uint8_t *>(c.workspace);
+  const uint64_t rows = uint64_t(c.num_rows), slots = 2 * uint64_t(p.grid);
+  p.head = reinterpret_cast<int32_t *>(ws);
+  ws += 16;
+  p.gpre = reinterpret_cast<int32_t *>(ws);
+  ws += align16(4 * rows);
+  p.gseq = reinterpret_cast<int32_t *>(ws);
+  ws += align16(4 * rows);
+  p.gpos = reinterpret_cast<int32_t *>(ws);
+  ws += align16(4 * rows + 4);
+  p.part_o = reinterpret_cast<uint16_t *>(ws);
+  p.part_sc = reinterpret_cast<float *>(p.part_o + slots * kCols * 512);
+  p.part_ml = reinterpret_cast<float2 *>(p.part_sc + slots * kCols * 8);
+  hipStream_t s = static_cast<hipStream_t>(c.stream);
+  if (!p.lds_plan) mla_chunk_plan_kernel<<<1, 1024, 0, s>>>(p);
+  const int grid = (p.grid + 7) / 8 * 8;  // XCD-contiguous shares need whole rounds
+  mla_chunk_kernel<<<grid, kThreads, 0, s>>>(p);
+  mla_chunk_merge_kernel<<<dim3(p.groups_max, kCols / 4), 256, 0, s>>>(p);
+}
+
+}  // namespace ifattn

@@ -50,6 +50,7 @@
 
 #include "common.h"
 #include "ifattn_internal.h"
+#include "mla_chunk.h"
 #include "mla_row_write.h"
 #include "split_k.h"
 
@@ -1660,6 +1661,16 @@ int32_t mla_run(const MlaCall &c, const char *what) {
   const uint64_t need = mla_workspace(c.num_rows, c.heads, sparse, c.topk, c.n_sinks);
   if (!c.workspace || c.workspace_bytes < need || !aligned16(c.workspace))
     return fail(IFATTN_EWORKSPACE, what, "workspace missing, short or misaligned");
+  if (c.fmt == kFmtBf16 && !sparse) {  // prompt chunks: many rows per staged key tile
+    const MlaChunkCall cc{c.q,       c.cache,  c.block_tables, c.table_stride, c.cu_q,       c.kv_lens,
+                          c.num_seqs, c.num_rows, c.window,     c.sink_k,       c.sink_v,     c.n_sinks,
+                          c.out,     c.heads,  c.block_size,   c.num_blocks,   c.max_context, c.scale,
+                          c.workspace, c.workspace_bytes, c.stream};
+    if (mla_chunk_takes(cc)) {
+      launch_mla_chunk(cc);
+      return launch_status(what);
+    }
+  }
   const uint64_t max_workers = mla_max_workers(sparse, c.num_rows, c.topk, c.n_sinks);
   if (max_workers > (uint64_t(1) << 28)) return fail(IFATTN_EINVAL, what, "too many rows for the work split");
   MlaParams p{};
@@ -1810,7 +1821,9 @@ extern "C" uint64_t ifattn_mla_attention_workspace_size(int32_t num_rows, int32_
   (void)max_context;
   (void)window;
   (void)block_size;
-  return mla_workspace(num_rows, heads, topk > 0, topk, n_sinks);
+  const uint64_t rows = mla_workspace(num_rows, heads, topk > 0, topk, n_sinks);
+  const uint64_t chunks = topk > 0 ? 0 : mla_chunk_workspace(num_rows);
+  return rows > chunks ? rows : chunks;
 }
 
 extern "C" int32_t ifattn_mla_window_attention_bf16(

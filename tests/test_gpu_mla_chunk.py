@@ -1,0 +1,125 @@
+"""MLA window attention of packed prompt chunks (two or more query rows per
+sequence on average) against the CPU oracle, bf16 outputs within 1e-2 abs +
+1e-2 rel: group edges (128 columns of (row, head)), tile and window edges,
+partial sink tiles, rows without keys, pieces split over workers, more groups
+than one workgroup plans in LDS, and graph replay."""
+import math
+
+import numpy as np
+import pytest
+
+import oracle
+from helpers import assert_close, bf16_host, bits_host, to_dev
+from ironpangu_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def make(seed, counts, kv, heads, bs, n_sinks, pad_blocks=0):
+    rng = np.random.default_rng(seed)
+    kv = np.asarray(kv, np.int32)
+    need = np.maximum((kv.astype(np.int64) + bs - 1) // bs, 1)
+    pool = int(need.sum()) + 8
+    table = W.block_tables_for(rng, np.maximum(kv, 1), bs, pool, int(need.max()) + pad_blocks)
+    cu = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    q = W.bf16_randn(rng, (int(cu[-1]), heads, 576), 0.5)
+    cache = W.bf16_randn(rng, (pool * bs, 576), 0.5)
+    sk = W.bf16_randn(rng, (n_sinks, 576), 0.5) if n_sinks else None
+    sv = W.bf16_randn(rng, (n_sinks, 512), 0.5) if n_sinks else None
+    return q, cache.reshape(pool, bs, 576), table, kv, cu, sk, sv
+
+
+def call(dev, window, max_context, out=None, workspace=None):
+    from ironpangu_amd import ops
+    q, cache, table, kv, cu, sk, sv = dev
+    return ops.mla_attention(q, cache, table, kv, max_context, cu_seqlens=cu, window=window,
+                             sink_keys=sk, sink_values=sv, out=out, workspace=workspace)
+
+
+def check(case, window):
+    import torch
+    q, cache, table, kv, cu, sk, sv = case
+    bs = cache.shape[1]
+    dev = [None if t is None else to_dev(t) for t in case]
+    max_context = table.shape[1] * bs
+    out = call(dev, window, max_context)
+    torch.cuda.synchronize()
+    exp = oracle.mla_attention(q, cache.reshape(-1, 576), table, kv, q.shape[1], bs,
+                               1 / math.sqrt(192.0), cu_seqlens=cu, window=window, sink_k=sk, sink_v=sv)
+    assert_close(bf16_host(out), exp)
+    return dev, max_context, out
+
+
+@pytest.mark.parametrize("heads", [1, 3, 6, 16])
+@pytest.mark.parametrize("window,bs,n_sinks", [(0, 16, 0), (37, 16, 128), (512, 32, 1), (0, 64, 33),
+                                               (100, 128, 0)])
+def test_chunk_shapes(heads, window, bs, n_sinks):
+    print(f"chunk heads={heads} window={window} bs={bs} sinks={n_sinks}", flush=True)
+    per = 128 // heads  # rows of one group
+    counts = [per, per + 1, 2, 1, 2 * per - 1, 40]
+    kv = [per, 700, 2, 333, 2 * per + 31, 1031]
+    check(make(heads + window, counts, kv, heads, bs, n_sinks, pad_blocks=1), window)
+
+
+def test_chunk_split_over_workers():
+    # One short chunk over a long context: a single group cut into many pieces,
+    # and a second one whose pieces cross the sink tiles.
+    check(make(3, [5, 8], [20011, 4097], 16, 16, 128), 0)
+
+
+def test_chunk_rows_without_keys():
+    # kv_len below the row count: the first rows see no key; an empty cache.
+    case = make(4, [20, 9], [7, 0], 6, 16, 0)
+    _, _, out = check(case, 64)
+    assert (bits_host(out)[:13] & 0x7FFF == 0).all() and (bits_host(out)[20:] & 0x7FFF == 0).all()
+
+
+def test_chunk_zero_row_sequences():
+    check(make(5, [0, 30, 0, 0, 17, 0], [50, 90, 16, 1, 400, 33], 16, 32, 17), 128)
+
+
+@pytest.mark.parametrize("n_sinks", [0, 20])
+def test_chunk_plan_launch(n_sinks):
+    # more than 512 groups (plan launch) and more than 512 sequences
+    rng = np.random.default_rng(6)
+    counts = rng.integers(1, 5, 700)
+    kv = counts + rng.integers(0, 60, 700)
+    assert counts.sum() >= 2 * len(counts)
+    check(make(7, counts.tolist(), kv, 4, 16, n_sinks), 33)
+
+
+def test_chunk_large_values_keep_their_range():
+    # Partials are fp16 under a power-of-two scale: latents far beyond fp16's
+    # range, split over many pieces, still give the oracle's output (relative
+    # bound; scores kept finite by a small q).
+    import torch
+    q, cache, table, kv, cu, sk, sv = make(8, [9], [6000], 16, 64, 0)
+    big = (W.bf16_to_f32(cache) * np.float32(2.0 ** 20)).astype(np.float32)
+    small = (W.bf16_to_f32(q) * np.float32(2.0 ** -20)).astype(np.float32)
+    cache, q = W.bf16_bits(big), W.bf16_bits(small)
+    dev = [to_dev(q), to_dev(cache), to_dev(table), to_dev(kv), to_dev(cu), None, None]
+    out = call(dev, 0, 6016)
+    torch.cuda.synchronize()
+    exp = oracle.mla_attention(q, cache.reshape(-1, 576), table, kv, 16, 64, 1 / math.sqrt(192.0),
+                               cu_seqlens=cu)
+    assert_close(bf16_host(out) * 2.0 ** -20, exp * 2.0 ** -20)
+
+
+def test_chunk_graph_replay():
+    import torch
+    case = make(9, [40, 3, 70], [900, 40, 70], 16, 16, 128)
+    dev, max_context, eager = check(case, 512)
+    out = torch.zeros_like(eager)
+    from ironpangu_amd import ops
+    n = ops.lib().ifattn_mla_attention_workspace_size(113, 16, max_context, 512, 0, 128, 16)
+    ws = torch.empty(int(n), dtype=torch.uint8, device="cuda")
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        call(dev, 512, max_context, out=out, workspace=ws)
+    for _ in range(3):
+        out.zero_()
+        ws.fill_(0xA5)
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), eager.view(torch.int16))
