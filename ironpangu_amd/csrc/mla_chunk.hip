@@ -64,7 +64,7 @@ constexpr int kStages = 3;
 #endif
 constexpr int kAhead = IFATTN_CHUNK_AHEAD;  // LDS operands in flight ahead of the MFMAs
 constexpr int kStart = 3;      // work units (tiles) charged per group: q loads and output stores
-constexpr int kMinShare = 8;   // smallest share, in tiles
+constexpr int kMinShare = 3;   // smallest share, in tiles (8: calls of 70 rows 48 us, now 31-39; 5: 39)
 constexpr int kLdsGroups = kThreads;  // calls of at most this many groups and sequences plan in LDS
 
 struct ChunkParams {

@@ -38,8 +38,8 @@
 // 1152 (three VALU ops per four codes instead of a convert per code), with q
 // in fp16 and the bias term removed per head. Row-quantized rows (576 int8 or
 // int4 codes and one fp32 scale per row, as if_cache_quantize writes them,
-// native/kernels/cache_quantization.cpp:12-38) are gathered row by row with
-// their scales staged behind the tile; keys are dequantized in registers to
+// native/kernels/cache_quantization.cpp:12-38) split the scores by keys instead
+// (mla_rq_item); keys are dequantized in registers to
 // the bf16 values if_cache_dequantize would write (the reference attends over
 // that dequantized cache, token_executor.h:806-822), V stays in codes with the
 // row scale folded into the probabilities. Rows split over several
@@ -81,7 +81,8 @@ struct MlaParams {
   int2 *row_slot;               // [rows] (first partial slot, slot count); (-1, 0): the row
                                 // writes its output directly
   int32_t *start_row;           // [max_workers] first row not wholly before each worker's share
-  uint16_t *part_o;             // [slots, heads, 512] bf16 O / l of each partial
+  uint16_t *part_o;             // [slots, heads, 512] O / l of each partial: bf16, or scaled fp16
+  float *part_sc;               // [slots, heads, 8] inverse scale of each 64 dims (fp16 partials)
   float *part_ml;               // [slots, heads, 2]
   int64_t num_blocks;
   uint32_t cache_bytes;  // sparse and row-quantized gathers: byte extent of the cache (< 4 GiB - 16)
@@ -380,9 +381,9 @@ template <int F>
 struct MlaRow {
   static constexpr uint32_t BYTES = F == kFmtC8 ? 656 : (F == kFmtRq8 ? 576 : (F == kFmtRq4 ? 288 : 1152));
   static constexpr uint32_t CHUNKS = BYTES / 16;  // 72, 41, 36 or 18
-  // Direct-to-LDS loads per wave per tile: 32 rows = 2304 (bf16), 1312 (C8),
-  // 1152 (Rq8) or 576 (Rq4) 16-byte chunks.
-  static constexpr int NI = F == kFmtC8 ? 6 : (F == kFmtRq8 ? 5 : (F == kFmtRq4 ? 3 : 9));
+  // Direct-to-LDS loads per wave per tile of the four-wave layout: 32 rows =
+  // 2304 (bf16) or 1312 (C8) 16-byte chunks.
+  static constexpr int NI = F == kFmtBf16 ? 9 : 6;
   static constexpr uint32_t SLOT = 4 * NI * 1024;  // LDS bytes per staged tile
   // LDS byte of 16-byte chunk j of tile row r. bf16 rows (1152 B: odd rows
   // start half a bank period in) XOR the latent chunk index with the row's low
@@ -399,8 +400,28 @@ struct MlaRow {
 static_assert(MlaRow<kFmtBf16>::NI * 4 * 64 == 32 * 72, "bf16 tile = 2304 chunks");
 static_assert(18 * 64 == 16 * 72, "bf16 loads 0..17 move exactly tile rows 0..15");
 static_assert(MlaRow<kFmtC8>::NI * 4 * 64 >= 32 * 41, "C8 tile fits the slot");
-static_assert(MlaRow<kFmtRq8>::NI * 4 * 64 >= 32 * 36 && MlaRow<kFmtRq4>::NI * 4 * 64 >= 32 * 18,
-              "row-quantized tiles fit the slot");
+
+// LDS of the row-quantized formats (mla_rq_item): two buffers of 64 keys, one
+// being read and one in flight, each holding the rows as stored and their
+// scales, then the probabilities.
+template <int F>
+struct MlaRq {
+  static constexpr int KEYS = 16 * kMlaWaves;
+  static constexpr uint32_t ROW = MlaRow<F>::BYTES;
+  static constexpr uint32_t SCALES = KEYS * ROW;
+  static constexpr uint32_t BUF = SCALES + 4 * KEYS;
+  static constexpr uint32_t PROB = 2 * BUF;
+  static constexpr uint32_t BYTES = PROB + KEYS * 16 * 2;
+  // The 16-byte chunks of a row are rotated by ROT(row) = row of 16 >> ROT_SHIFT,
+  // so that the 16 rows of a score read (one instruction reads the same dims of
+  // all of them) start on 16 different bank groups: unrotated rows (36 or 18
+  // chunks, against 16 per bank period) share 4 or 8.
+  static constexpr int CHUNKS = int(ROW / 16);
+  static constexpr int ROT_SHIFT = F == kFmtRq8 ? 2 : 3;
+  // Direct-to-LDS loads per wave per buffer: its 16 rows and their scales.
+  static constexpr int ROWS_NI = int((16 * ROW + 1023) / 1024);
+  static constexpr int NI = ROWS_NI + 1;
+};
 
 // Ring depth and persistent workgroups per CU of each kernel variant. bf16
 // runs one workgroup of four waves per CU with a 4-tile ring (its 36-KB tiles
@@ -412,16 +433,16 @@ static_assert(MlaRow<kFmtRq8>::NI * 4 * 64 >= 32 * 36 && MlaRow<kFmtRq4>::NI * 4
 // 95.9 us with one workgroup and 6 stages, 75.9 us with two and 2 stages.
 template <int F, bool SPARSE, bool WIDE = false>
 struct MlaCfg {
-  static constexpr bool C8 = mla_int(F);
-  // Dense integer formats run three workgroups per CU (three waves per SIMD):
-  // ring slots of exactly the 1-KiB loads a tile needs (21 for a 20992-B C8
-  // tile) and one score buffer (two barriers per tile) fit three in the LDS,
-  // and the tile math of one workgroup hides behind the other two (config-5
-  // shapes 380-386 -> 349-356 us against two workgroups with double score
-  // buffers). Sparse C8 keeps two: three (with 512-entry slot lists) measured
-  // 81 against 72 us on top-2048, and two with 3-slot rings of 21-KiB slots and
-  // one score buffer 74 us. Row-quantized slots end with the tile's 32 row
-  // scales (256 bytes: the direct-to-LDS scale load writes a dword per lane).
+  static constexpr bool C8 = F == kFmtC8;
+  static constexpr bool RQ = mla_rq(F);
+  // Dense C8 runs three workgroups per CU (three waves per SIMD): ring slots
+  // of exactly the 1-KiB loads a tile needs (21 for a 20992-B C8 tile) and one
+  // score buffer (two barriers per tile) fit three in the LDS, and the tile
+  // math of one workgroup hides behind the other two (config-5 shapes 380-386
+  // -> 349-356 us against two workgroups with double score buffers). Sparse C8
+  // keeps two: three (with 512-entry slot lists) measured 81 against 72 us on
+  // top-2048, and two with 3-slot rings of 21-KiB slots and one score buffer 74
+  // us. Row-quantized rows run two (mla_rq_item).
   static constexpr bool TIGHT = C8 && !SPARSE;
   // Dense bf16 calls of at least 2^18 keys (WIDE) run two workgroups per CU,
   // each with a 2-slot ring and one score buffer (exactly 160 KiB): config-5
@@ -429,14 +450,8 @@ struct MlaCfg {
   // while one workgroup runs a sink block, the other keeps streaming)
   // 0.0735-0.0773 -> 0.0716-0.0753 ms. Smaller calls keep one workgroup with a
   // 4-slot ring and plan for themselves.
-  static constexpr bool B2 = !C8 && !SPARSE && WIDE;
-  // Row-quantized int8 tiles run two workgroups with 3-slot rings: their
-  // gather addressing, bf16 dequantization and the rope codes' extra MFMAs
-  // need more than the 168 registers of three workgroups (they spilled 17 and
-  // ran 0.514-0.520 against 0.488-0.490 ms on config-5 rows). Int4 tiles (9 KB)
-  // run three with 2-slot rings: 0.438-0.441 against 0.471-0.472 ms despite 8
-  // spilled registers.
-  static constexpr int WGS = F == kFmtRq8 ? 2 : (F == kFmtRq4 ? 3 : (C8 ? ((TIGHT && !SPARSE) ? 3 : 2) : (B2 ? 2 : 1)));
+  static constexpr bool B2 = F == kFmtBf16 && !SPARSE && WIDE;
+  static constexpr int WGS = TIGHT ? 3 : (C8 || RQ || B2 ? 2 : 1);
   // Waves per workgroup. Eight waves with 64-dim slices measured slower for
   // bf16 (612 against 532 us on 128 rows of log-uniform [1024, 65536] keys):
   // the score exchange then sums eight partials per tile.
@@ -447,28 +462,28 @@ struct MlaCfg {
 #ifndef IFATTN_MLA_BF16_XB
 #define IFATTN_MLA_BF16_XB 1
 #endif
-  static constexpr int STAGES = F == kFmtRq8 ? 3 : F == kFmtRq4 ? 2 : (C8 ? 2 : (SPARSE ? 3 : (B2 ? 2 : IFATTN_MLA_BF16_STAGES)));
+  static constexpr int STAGES = C8 ? 2 : (SPARSE ? 3 : (B2 ? 2 : IFATTN_MLA_BF16_STAGES));
   // 1-KiB loads per tile
   static constexpr int LOADS = TIGHT ? int((32 * MlaRow<F>::BYTES + 1023) / 1024) : 4 * MlaRow<F>::NI;
-  static constexpr int SCALES = mla_rq(F) ? LOADS * 1024 : 0;  // LDS byte of the row scales
-  static constexpr int SLOT = TIGHT ? LOADS * 1024 + (mla_rq(F) ? 256 : 0) : int(MlaRow<F>::SLOT);
+  static constexpr int SLOT = TIGHT ? LOADS * 1024 : int(MlaRow<F>::SLOT);
   static constexpr int XB = (TIGHT || B2) ? 1 : (!C8 && !SPARSE ? IFATTN_MLA_BF16_XB : 2);  // score buffers
-  static constexpr int RING = SLOT * STAGES;
+  static constexpr int RING = RQ ? int(MlaRq<F>::BYTES) : SLOT * STAGES;
+  // Score exchange rows: inside the ring for the row-quantized layout (only
+  // its sink blocks use it, between items).
+  static constexpr int XBUF = RQ ? 0 : XB * NW * 64;
   // (+ the self-plan arrays: two ints per planned row, except the wide variant)
-  static constexpr int LDS = RING + XB * NW * 64 * 32 + (SPARSE ? 4 * kSparsePart : 0) +
+  static constexpr int LDS = RING + XBUF * 32 + (RQ ? 4 * 64 + 16 : 0) + (SPARSE ? 4 * kSparsePart : 0) +
                              (B2 ? 0 : 2 * 4 * 64 * kMlaWaves + 64);
   static_assert(LDS * WGS <= 160 * 1024, "LDS per CU");
-  static_assert(!mla_rq(F) || !SPARSE, "row-quantized rows are attended densely");
-  // Waves that issue NI loads per tile (the rest issue NI - 1; with row
-  // scales, the last wave issues the scale load on top of its NI - 1).
+  static_assert(!RQ || RING >= NW * 64 * 32, "the sinks' score exchange fits the ring");
+  static_assert(!RQ || !SPARSE, "row-quantized rows are attended densely");
+  // Waves that issue NI loads per tile (the rest issue NI - 1).
   static constexpr int FULL_WAVES = TIGHT ? LOADS - 4 * (MlaRow<F>::NI - 1) : 4;
-  static_assert(!mla_rq(F) || FULL_WAVES < 4, "the scale load goes to a wave with NI - 1 loads");
 };
 // Persistent workgroups per CU of the kernel variant a call runs (the grid is
 // that many per CU, all resident at once).
 inline int wgs_mla(int fmt, bool sparse, bool wide) {
-  if (fmt == kFmtRq8) return MlaCfg<kFmtRq8, false>::WGS;
-  if (fmt == kFmtRq4) return MlaCfg<kFmtRq4, false>::WGS;
+  if (fmt == kFmtRq8 || fmt == kFmtRq4) return MlaCfg<kFmtRq8, false>::WGS;
   if (fmt != kFmtBf16) return sparse ? MlaCfg<kFmtC8, true>::WGS : MlaCfg<kFmtC8, false>::WGS;
   return sparse ? MlaCfg<kFmtBf16, true>::WGS
                 : (wide ? MlaCfg<kFmtBf16, false, true>::WGS : MlaCfg<kFmtBf16, false>::WGS);
@@ -487,6 +502,38 @@ struct MlaGeo {
 };
 
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;  // sparse slot list: no key
+
+// A lane's N consecutive dims of a partial's O / l (o times inv). Row-quantized
+// rows (F16) hold them in fp16 under a power-of-two scale over the four lanes (g)
+// that share the wave's dims: the bytes of bf16 with 2^-11 of the largest value
+// as the worst rounding instead of 2^-8 of each, which their large rows need to
+// stay within the outputs' bound (a split of the call into other shares moved
+// one past it). The other formats hold bf16 (the scale costs the small window
+// and sparse calls 1-3%). Returns the inverse scale.
+template <bool F16, int N>
+__device__ __forceinline__ float mla_store_partial(uint16_t *po, const float (&o)[N], float inv) {
+  if constexpr (!F16) {
+#pragma unroll
+    for (int k = 0; k < N; k += 8)
+      store_u32x4(po + k, u32x4{pack_bf16x2(o[k] * inv, o[k + 1] * inv),
+                                pack_bf16x2(o[k + 2] * inv, o[k + 3] * inv),
+                                pack_bf16x2(o[k + 4] * inv, o[k + 5] * inv),
+                                pack_bf16x2(o[k + 6] * inv, o[k + 7] * inv)});
+    return 1.0f;
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) amax = fmaxf(amax, fabsf(o[i]));
+  const float ps = f16_range_scale(max_xor32(max_xor16(amax * inv)));
+  const float f = inv * ps;
+  auto two = [&](int i) {
+    const f16x2 h = __builtin_convertvector((f32x2{o[i] * f, o[i + 1] * f}), f16x2);
+    return __builtin_bit_cast(uint32_t, h);
+  };
+#pragma unroll
+  for (int k = 0; k < N; k += 8) store_u32x4(po + k, u32x4{two(k), two(k + 2), two(k + 4), two(k + 6)});
+  return __uint_as_float((254u << 23) - __float_as_uint(ps));  // 1 / ps
+}
 
 __device__ __forceinline__ int mla_tile_token(int g, int j) {
   return j < 4 ? 4 * g + j : 16 + 4 * g + (j - 4);
@@ -658,8 +705,8 @@ template <int F, bool SPARSE, bool WIDE>
 __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, float (*xbuf)[8],
                                          uint32_t *slot_list, int row, const MlaSpan &sp, int j0,
                                          int j1, int slot, int w, int lane) {
-  constexpr bool C8 = mla_int(F);  // integer latent codes (C8 or row-quantized)
-  constexpr bool RQ = mla_rq(F);
+  constexpr bool C8 = mla_int(F);
+  static_assert(!mla_rq(F), "row-quantized rows run mla_rq_item");
   using R = MlaRow<F>;
   using Cfg = MlaCfg<F, SPARSE, WIDE>;
   constexpr int S = Cfg::STAGES;
@@ -739,9 +786,8 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
   // C8 rows: the latent QK^T runs in fp16 on the biased codes (code +
   // kI8Bias, exact); the wave's q slice is scaled per head by a power of two
   // into fp16 range, and kI8Bias * sum(q slice) leaves each partial score.
-  // (Row-quantized keys are dequantized to bf16 instead; see score().)
   float k_corr = 0.0f, q_unscale = 1.0f;
-  if constexpr (C8 && !RQ) {
+  if constexpr (C8) {
     float amax = 0.0f;
 #pragma unroll
     for (int s = 0; s < KS; ++s) amax = fmaxf(amax, bf16x8_absmax(qv[s]));
@@ -784,36 +830,6 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
         const uint32_t slot = r < 32u && t0 + int(r) < t_end ? slot_list[ti * kMlaTile + r] : kNoRow;
         const uint32_t off = slot == kNoRow ? 0xFFFFFFF0u : slot * R::BYTES + lcol[k];
         lds_dma16(rc, off, dst + uint32_t(k) * 4096);
-      }
-    } else if constexpr (RQ) {
-      // Row-quantized rows: every lane gathers its chunk's row through the
-      // block window (any page size; rows outside [t_begin, t_end) land as
-      // zeros), and the last wave loads the tile's 32 row scales behind the rows.
-      const int lower = t_begin > t0 ? t_begin - t0 : 0;
-      const int upper = t_end - t0 < kMlaTile ? t_end - t0 : kMlaTile;
-      if (((t0 + kMlaTile - 1) >> bs_log2) - wblk0 >= 64) {
-        wblk0 = t0 >> bs_log2;
-        load_window();
-      }
-      const u32x4 rc = raw_rsrc(p.cache, p.cache_bytes);
-      auto row_slot = [&](int r) {  // physical row of tile row r (all lanes take part)
-        const int pos = t0 + r;
-        const int blk = __shfl(lane_blocks, ((pos >> bs_log2) - wblk0) & 63, 64);
-        return uint32_t(blk) * uint32_t(bs) + uint32_t(pos & (bs - 1));
-      };
-#pragma unroll
-      for (int k = 0; k < R::NI; ++k) {
-        if (4 * k + w >= Cfg::LOADS) break;
-        const int r = int(lrow[k]);
-        const uint32_t srow = row_slot(r & 31);
-        const uint32_t off = r >= lower && r < upper ? srow * R::BYTES + lcol[k] : 0xFFFFFFF0u;
-        lds_dma16(rc, off, dst + uint32_t(k) * 4096);
-      }
-      if (w == 3) {
-        const uint32_t srow = row_slot(lane & 31);
-        const uint32_t off = lane < 32 && lane >= lower && lane < upper ? srow * 4u : 0xFFFFFFF0u;
-        lds_dma4(raw_rsrc(p.row_scales, p.scale_bytes), off,
-                 ring_base + uint32_t(ti % S) * Cfg::SLOT + uint32_t(Cfg::SCALES));
       }
     } else {
       const int lower = t_begin > t0 ? t_begin - t0 : 0;  // rows before the window start
@@ -875,28 +891,10 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
       live = (upper >= 32 ? 0xFFFFFFFFu : ((1u << upper) - 1u)) & ~((1u << lower) - 1u);
     }
     // K operand: token 16mt + c, latent dims DPW w + 32s + 8g (+ rope dims 32(w&1) + 8g).
-    // Row-quantized keys become the bf16 values if_cache_dequantize writes,
-    // bf16(code * scale) (cache_quantization.cpp:39-57): a score depends on
-    // that rounding (a large-scale row moves by up to a percent without it),
-    // so the keys are scored exactly as the reference's dequantized cache.
     u32x4 k[2][KS + 1];
 #pragma unroll
     for (int mt = 0; mt < 2; ++mt) {
       const uint32_t r = uint32_t(16 * mt + c);
-      if constexpr (RQ) {
-        const float rs = *reinterpret_cast<const float *>(tile + Cfg::SCALES + 4 * r);
-        auto codes = [&](uint32_t dim) {  // 8 codes of dims dim .. dim + 7
-          if constexpr (F == kFmtRq4)
-            return i4x8_to_i8x8(*reinterpret_cast<const uint32_t *>(tile + r * R::BYTES + dim / 2));
-          else
-            return *reinterpret_cast<const u32x2 *>(tile + r * R::BYTES + dim);
-        };
-#pragma unroll
-        for (int s = 0; s < KS; ++s) k[mt][s] = i8x8_dequant_bf16(codes(uint32_t(DPW * w + 32 * s + 8 * g)), rs);
-        k[mt][KS] = w < 2 ? i8x8_dequant_bf16(codes(uint32_t(512 + 32 * (w & 1) + 8 * g)), rs)
-                          : u32x4{0, 0, 0, 0};
-        continue;
-      }
 #pragma unroll
       for (int s = 0; s < KS; ++s) {
         if constexpr (C8) {
@@ -919,18 +917,7 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const uint32_t r = uint32_t(mla_tile_token(g, j));
-      if constexpr (RQ) {
-        static_assert(EPL == 8, "row-quantized V operands are 8 dims per lane");
-        if constexpr (F == kFmtRq4) {
-          const u32x2 x = i4x8_to_i8x8(
-              *reinterpret_cast<const uint32_t *>(tile + r * R::BYTES + (DPW * w + 8 * c) / 2));
-          v[j] = u32x4{x[0], x[1], 0u, 0u};
-        } else {
-          const u32x2 x = *reinterpret_cast<const u32x2 *>(tile + r * R::BYTES + DPW * w + 8 * c);
-          v[j] = u32x4{x[0], x[1], 0u, 0u};
-        }
-        sk[j] = *reinterpret_cast<const float *>(tile + Cfg::SCALES + 4 * r);
-      } else if constexpr (C8) {
+      if constexpr (C8) {
         if constexpr (EPL == 8) {
           const u32x2 x = *reinterpret_cast<const u32x2 *>(tile + r * R::BYTES + DPW * w + 8 * c);
           v[j] = u32x4{x[0], x[1], 0u, 0u};
@@ -949,8 +936,7 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
       }
     }
 
-    // Row-quantized keys were dequantized above: bf16 scores, no scale.
-    mla_tile_scores<C8 && !RQ, NW>(k, sk, qv, xb, w, lane, k_corr, q_unscale);
+    mla_tile_scores<C8, NW>(k, sk, qv, xb, w, lane, k_corr, q_unscale);
   };
 
   // Ring: tile ti lives in slot ti % S; tiles 0..S-1 are issued up front. In
@@ -963,9 +949,8 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
 #pragma unroll
   for (int i = 0; i < S; ++i)
     if (i < n_tiles) issue(i);
-  // Loads per wave per tile: NI, or NI - 1 for the waves past LOADS (the
-  // scale load brings the last wave of a row-quantized tile back to NI).
-  const bool full_loads = !Cfg::TIGHT || w < Cfg::FULL_WAVES || (RQ && w == 3);
+  // Loads per wave per tile: NI, or NI - 1 for the waves past LOADS.
+  const bool full_loads = !Cfg::TIGHT || w < Cfg::FULL_WAVES;
   if (S - 1 < n_tiles) {  // tile 0; tiles 1 .. S-1 may stay in flight
     if (full_loads)
       lds_dma_wait<(S - 1) * R::NI>();
@@ -1018,20 +1003,270 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
                                     pack_bf16x2(v[6] * inv, v[7] * inv)});
     }
   } else {
-    // Partials store O / l in bf16 (half the partial traffic; the merge
-    // weighs them by l), (m, l) in fp32.
     const int64_t prow = int64_t(slot) * p.heads + c;
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    uint16_t *po = p.part_o + prow * DV + d0;
-#pragma unroll
-    for (int k = 0; k < EPL / 2; ++k) {
-      const float *v = ov + 8 * k;
-      store_u32x4(po + 8 * k, u32x4{pack_bf16x2(v[0] * inv, v[1] * inv),
-                                    pack_bf16x2(v[2] * inv, v[3] * inv),
-                                    pack_bf16x2(v[4] * inv, v[5] * inv),
-                                    pack_bf16x2(v[6] * inv, v[7] * inv)});
-    }
+    mla_store_partial<false>(p.part_o + prow * DV + d0, ov, inv);
     if (w == 0 && g == 0) *reinterpret_cast<float2 *>(p.part_ml + prow * 2) = make_float2(acc.m, l_tot);
+  }
+}
+
+// Item of the row-quantized formats: tiles [j0, j1) of row `row` (span sp);
+// output, or partial slot `slot` when slot >= 0.
+//
+// Four waves, two workgroups per CU, steps of 64 keys. Scores are split by
+// keys: wave w scores keys [16w, 16w + 16) of a step over all 576 dims (q in 72
+// registers), so no partial scores are exchanged and every exponential is
+// computed once (waves that split the dims, as for the other formats, exchange
+// 32 bytes of scores per lane and 32 keys and each repeat the softmax). PV is
+// split by dims (wave w owns latent dims [128w, 128w + 128) of all the step's
+// keys); the probabilities go through LDS in MFMA operand layout. A wave's 16
+// rows are contiguous in the cache and are copied as they lie.
+//
+// Two barriers a step: one publishes P (and every wave's rows), one retires the
+// buffer for the step after next, whose loads are then in flight for a whole
+// step. The running max lags a step: P is taken against the max of the earlier
+// steps (any base is exact in floating point while exponents stay small), the
+// waves publish their keys' maxima beside it, and all of them move to the new
+// base after PV. An item's first step, and a step whose scores exceed the base
+// by 2^64, instead share the maxima before P is used.
+//
+// Bound: VALU, 694 instructions per wave and 64 keys (about 360 dequantize the
+// wave's keys, 192 convert V), each SIMD's VALU busy 69% of the time; the row
+// loads alone take 0.2 ms of the int8 call below. int8 rows, 128 sequences of
+// 1024..65536 keys: 0.363 -> 0.262 ms (0.277 with unrotated rows, whose score
+// reads kept the LDS in bank conflicts half the time); int4 rows 0.345 -> 0.303 ms.
+// Eight waves with 128-key steps in one workgroup per CU ran 0.321 ms: the
+// phases of a step then wait for each other with nothing beside them.
+template <int F>
+__device__ __forceinline__ void mla_rq_item(const MlaParams &p, uint8_t *ring, float (*s_max)[16],
+                                            int *s_over, int row, const MlaSpan &sp, int j0, int j1,
+                                            int slot, int w, int lane) {
+  using L = MlaRq<F>;
+  constexpr uint32_t ROW = L::ROW;
+  const int c = lane & 15, g = lane >> 4;
+  const bool head_live = c < p.heads;
+
+  // q: dims 32s + 8g (s < 18); padded heads read zeros.
+  u32x4 qv[18];
+  {
+    const auto rq = make_rsrc(p.q + int64_t(row) * p.heads * 576, uint32_t(p.heads) * 576 * 2);
+    const uint32_t qh = head_live ? uint32_t(c) * 576 * 2 : 0x80000000u;
+#pragma unroll
+    for (int s = 0; s < 18; ++s) qv[s] = buf_load_x4(rq, qh + uint32_t(32 * s + 8 * g) * 2);
+  }
+  const int tile0 = uniform(sp.base + j0 * kMlaTile);
+  const int t_begin = uniform(sp.lo > tile0 ? sp.lo : tile0);
+  const int t_end = uniform(sp.hi < sp.base + j1 * kMlaTile ? sp.hi : sp.base + j1 * kMlaTile);
+  const int steps = (t_end - tile0 + L::KEYS - 1) / L::KEYS;
+  const int num_blocks = int(p.num_blocks);  // below 2^32 / 288 (4-GiB caches)
+  const int bs = p.block_size, bs_log2 = __builtin_ctz(uint32_t(p.block_size));
+  // Block ids of a 64-block window, one per lane (entries past the keys read 0).
+  int wblk0 = tile0 >> bs_log2, lane_blocks;
+  const auto rw = make_rsrc(p.block_tables + int64_t(sp.seq) * p.table_stride,
+                            uint32_t((t_end - 1) / bs + 1) * 4);
+  auto load_window = [&]() __attribute__((always_inline)) {
+    const int b = int(buf_load_x1(rw, uint32_t(wblk0 + lane) * 4));
+    lane_blocks = b < 0 ? 0 : (b >= num_blocks ? num_blocks - 1 : b);
+  };
+  load_window();
+
+  const uint32_t lds = lds_addr(ring);
+  const uint8_t *const cache = p.cache;
+  const float *const row_scales = p.row_scales;
+  // The wave moves its own 16 keys of step st (16-aligned positions: one
+  // block). The buffer base sits at the first live row; earlier rows' offsets
+  // wrap past the extent and land as zeros, like rows past the end.
+  uint32_t src[L::ROWS_NI];
+#pragma unroll
+  for (int n = 0; n < L::ROWS_NI; ++n) {
+    const int l = n * 64 + lane, r = l / L::CHUNKS, at = l % L::CHUNKS, j = at - (r >> L::ROT_SHIFT);
+    src[n] = uint32_t(r) * ROW + 16u * uint32_t(j < 0 ? j + L::CHUNKS : j);
+  }
+  auto issue = [&](int st) __attribute__((always_inline)) {
+    const int p0 = tile0 + st * L::KEYS + 16 * w;
+    const int lo = t_begin - p0, hi = t_end - p0;
+    const int a = lo < 0 ? 0 : (lo > 16 ? 16 : lo), b = hi < 0 ? 0 : (hi > 16 ? 16 : hi);
+    int at = (p0 >> bs_log2) - wblk0;
+    if (at >= 64 && b > a) {
+      wblk0 += at;
+      load_window();
+      // Wait here, with a wait the compiler accounts for: it would otherwise
+      // drain the loads in flight at every readlane below.
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      at = 0;
+    }
+    const int blk = __builtin_amdgcn_readlane(lane_blocks, at & 63);
+    const int64_t tok = int64_t(blk) * bs + (p0 & (bs - 1)) + a;
+    const uint32_t live = b > a ? uint32_t(b - a) : 0u, skip = uint32_t(a);
+    const u32x4 rs = raw_rsrc(cache + tok * ROW, live * ROW);
+    const uint32_t buf = lds + uint32_t(st & 1) * L::BUF;
+#pragma unroll
+    for (int n = 0; n < L::ROWS_NI; ++n)
+      if (uint32_t(n + 1) * 1024u <= 16 * ROW || lane < int(16 * ROW % 1024 / 16))
+        lds_dma16(rs, src[n] - skip * ROW,
+                  buf + uint32_t(w) * (16 * ROW) + uint32_t(n) * 1024u);
+    if (lane < 16)
+      lds_dma4(raw_rsrc(row_scales + tok, live * 4u), uint32_t(lane) * 4u - skip * 4u,
+               buf + L::SCALES + uint32_t(w) * 64u);
+  };
+
+  // q and the block ids have arrived before the first tile load: a wait for q
+  // inside the loop would drain the loads in flight at every step.
+  __builtin_amdgcn_s_waitcnt(0x0F70);
+  issue(0);
+  if (steps > 1) issue(1);
+
+  f32x4 acc[8];
+#pragma unroll
+  for (int b = 0; b < 8; ++b) acc[b] = f32x4{0, 0, 0, 0};
+  float m_run = -INFINITY, l_run = 0.0f;
+
+  // Score MFMA row m is key 4(m & 3) + (m >> 2) of the wave's 16, so that a
+  // lane's scores r are keys 4r + g and the four lane groups' PV reads of one
+  // instruction lie in consecutive rows (distinct banks).
+  const int krow16 = 4 * (c & 3) + (c >> 2), krow = 16 * w + krow16;
+  const int krot = krow16 >> L::ROT_SHIFT;
+  // Latent chunks never wrap (the last is CHUNKS - 5 or CHUNKS - 3); rope chunks do.
+  const uint32_t k_at = uint32_t(krow) * ROW + 16u * uint32_t(krot) + (F == kFmtRq8 ? 8u : 4u) * uint32_t(g);
+  uint32_t k_rope[2];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int byte = F == kFmtRq8 ? 512 + 32 * s + 8 * g : 256 + 16 * s + 4 * g;
+    const int j = byte / 16 + krot;
+    k_rope[s] = uint32_t(krow) * ROW + 16u * uint32_t(j >= L::CHUNKS ? j - L::CHUNKS : j) + uint32_t(byte % 16);
+  }
+
+  for (int st = 0; st < steps; ++st) {
+    const uint8_t *buf = ring + uint32_t(st & 1) * L::BUF;
+    if (st + 1 < steps)
+      lds_dma_wait<L::NI>();  // this step's rows; the next step's stay in flight
+    else
+      lds_dma_wait<0>();
+    // Scores of keys 16w + 4r + g (r < 4) for head c. The wave reads only rows
+    // that it moved itself: no barrier. Keys become the bf16 values
+    // if_cache_dequantize writes, bf16(code * scale) (cache_quantization.cpp:39-57):
+    // a score depends on that rounding (a large-scale row moves by up to a
+    // percent without it), so the keys are scored exactly as the reference's
+    // dequantized cache.
+    const float rs = *reinterpret_cast<const float *>(buf + L::SCALES + uint32_t(krow) * 4u);
+    f32x4 s0 = {0, 0, 0, 0}, s1 = {0, 0, 0, 0};
+#pragma unroll
+    for (int s = 0; s < 18; ++s) {
+      u32x2 k;
+      if constexpr (F == kFmtRq8)
+        k = *reinterpret_cast<const u32x2 *>(buf + (s < 16 ? k_at + 32 * s : k_rope[s & 1]));
+      else
+        k = i4x8_to_i8x8(*reinterpret_cast<const uint32_t *>(buf + (s < 16 ? k_at + 16 * s : k_rope[s & 1])));
+      const u32x4 kd = i8x8_dequant_bf16(k, rs);
+      if (s & 1) s1 = mfma16x16x32(kd, qv[s], s1);
+      else s0 = mfma16x16x32(kd, qv[s], s0);
+    }
+    float x[4], sk[4];
+    const int key0 = tile0 + st * L::KEYS + 16 * w + g;
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      sk[r] = *reinterpret_cast<const float *>(buf + L::SCALES + uint32_t(16 * w + 4 * r + g) * 4u);
+      x[r] = key0 + 4 * r >= t_begin && key0 + 4 * r < t_end ? (s0[r] + s1[r]) * p.scale_log2 : -INFINITY;
+      tmax = fmaxf(tmax, x[r]);
+    }
+    tmax = max_xor32(max_xor16(tmax));
+    if (g == 0) s_max[w][c] = tmax;
+    float pr[4];
+    auto probs = [&]() __attribute__((always_inline)) {
+      const float base = m_run == -INFINITY ? 0.0f : m_run;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pr[r] = fast_exp2(x[r] - base);
+      // k-step w >> 1, operand elements j < 4 (even wave) or j >= 4 (odd).
+      *reinterpret_cast<u32x2 *>(ring + L::PROB + uint32_t(w >> 1) * 1024u + lane * 16 + (w & 1) * 8) =
+          u32x2{pack_bf16x2(pr[0] * sk[0], pr[1] * sk[1]), pack_bf16x2(pr[2] * sk[2], pr[3] * sk[3])};
+    };
+    auto step_max = [&]() __attribute__((always_inline)) {
+      return fmaxf(fmaxf(s_max[0][c], s_max[1][c]), fmaxf(s_max[2][c], s_max[3][c]));
+    };
+    auto rebase = [&](float mx) __attribute__((always_inline)) {
+      const float m_new = fmaxf(m_run, mx);
+      const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int b = 0; b < 8; ++b) acc[b] *= alpha;
+    };
+    if (st == 0) {
+      __syncthreads();
+      rebase(step_max());
+    } else if (__any(tmax > m_run + 64.0f)) {
+      if (lane == 0) *s_over = 1;
+    }
+    probs();
+    __syncthreads();  // P, the maxima and every wave's rows
+    const float mx = step_max();
+    if (uniform(*s_over)) {
+      rebase(mx);
+      __syncthreads();  // every wave has seen the flag and the P it replaces
+      if (w == 0 && lane == 0) *s_over = 0;
+      probs();
+      __syncthreads();
+    }
+    l_run += (pr[0] + pr[1]) + (pr[2] + pr[3]);
+
+    // PV: 32 keys at a time, elements j of the operand: keys 32kk + 16(j >> 2)
+    // + 4(j & 3) + g; MFMA b, row m is dim 128w + 8m + b.
+#pragma unroll
+    for (int kk = 0; kk < 2; ++kk) {
+      if (kk > 0 && t_end - (tile0 + st * L::KEYS) <= 32) break;
+      const u32x4 pb = load_u32x4(ring + L::PROB + uint32_t(kk) * 1024u + uint32_t(lane) * 16u);
+      u32x2 v[8];  // eight codes (dims 128w + 8c ..) per key
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint8_t *vp = buf + uint32_t(32 * kk + 16 * (j >> 2) + 4 * (j & 3) + g) * ROW +
+                            16 * ((4 * (j & 3)) >> L::ROT_SHIFT);
+        if constexpr (F == kFmtRq8)
+          v[j] = *reinterpret_cast<const u32x2 *>(vp + 128 * w + 8 * c);
+        else
+          v[j] = i4x8_to_i8x8(*reinterpret_cast<const uint32_t *>(vp + 64 * w + 4 * c));
+      }
+#pragma unroll
+      for (int b = 0; b < 8; ++b) {
+        const int h = b >> 2, y = b & 3;
+        const u32x4 a = {mla_i8pair(mla_i8(v[0][h], y), mla_i8(v[1][h], y)),
+                         mla_i8pair(mla_i8(v[2][h], y), mla_i8(v[3][h], y)),
+                         mla_i8pair(mla_i8(v[4][h], y), mla_i8(v[5][h], y)),
+                         mla_i8pair(mla_i8(v[6][h], y), mla_i8(v[7][h], y))};
+        acc[b] = mfma16x16x32(a, pb, acc[b]);
+      }
+    }
+    if (__any(mx > m_run + 8.0f)) rebase(mx);
+    __syncthreads();  // every wave is done with this buffer, P and the maxima
+    if (st + 2 < steps) issue(st + 2);
+  }
+
+  // The waves' sums (each over its own keys).
+  const float l_own = sum_xor32(sum_xor16(l_run));
+  if (g == 0) s_max[w][c] = l_own;
+  __syncthreads();
+  const float l_tot = (s_max[0][c] + s_max[1][c]) + (s_max[2][c] + s_max[3][c]);
+  if (!head_live) return;
+  // Rows 4g + r of MFMA b: dims 128w + 32g + 8r + b, 32 consecutive per lane.
+  const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+  float ov[32];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int b = 0; b < 8; ++b) ov[8 * r + b] = acc[b][r];
+  if (slot < 0) {
+    uint16_t *op = p.out + (int64_t(row) * p.heads + c) * 512 + 128 * w + 32 * g;
+#pragma unroll
+    for (int k = 0; k < 32; k += 8)
+      store_u32x4(op + k, u32x4{pack_bf16x2(ov[k] * inv, ov[k + 1] * inv),
+                                pack_bf16x2(ov[k + 2] * inv, ov[k + 3] * inv),
+                                pack_bf16x2(ov[k + 4] * inv, ov[k + 5] * inv),
+                                pack_bf16x2(ov[k + 6] * inv, ov[k + 7] * inv)});
+  } else {
+    const int64_t prow = int64_t(slot) * p.heads + c;
+    const float sc = mla_store_partial<true>(p.part_o + prow * 512 + 128 * w + 32 * g, ov, inv);
+    if (g == 0) *reinterpret_cast<float2 *>(p.part_sc + prow * 8 + 2 * w) = make_float2(sc, sc);
+    if (w == 0 && g == 0) *reinterpret_cast<float2 *>(p.part_ml + prow * 2) = make_float2(m_run, l_tot);
   }
 }
 
@@ -1040,7 +1275,7 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
 // cache keys, four waves per row, heads in the MFMA N dimension. The (m, l, O)
 // partial of the sinks alone goes to the row's first partial slot. Runs as the
 // event at the start of the row's work units, in the share that holds it.
-template <int NW, bool DB>
+template <int NW, bool DB, bool F16>
 __device__ __forceinline__ void mla_sink_item(const MlaParams &p, float (*xbuf)[8], int row, int slot0,
                                               int w, int lane) {
   using Geo = MlaGeo<NW>;
@@ -1116,13 +1351,15 @@ __device__ __forceinline__ void mla_sink_item(const MlaParams &p, float (*xbuf)[
   if (!head_live) return;
   const int64_t prow = int64_t(slot0) * p.heads + c;  // the row's first slot
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-  uint16_t *po = p.part_o + prow * 512 + DPW * w + 4 * EPL * g;
+  float ov[4 * EPL];  // dims EPL r + b of the lane's run
 #pragma unroll
-  for (int k = 0; k < EPL; ++k) {
-    const int r = (4 * k) / EPL, b = (4 * k) % EPL;  // dims EPL r + b .. + 3 of the lane's run
-    *reinterpret_cast<u32x2 *>(po + 4 * k) =
-        u32x2{pack_bf16x2(acc.o[b][r] * inv, acc.o[b + 1][r] * inv),
-              pack_bf16x2(acc.o[b + 2][r] * inv, acc.o[b + 3][r] * inv)};
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int b = 0; b < EPL; ++b) ov[EPL * r + b] = acc.o[b][r];
+  const float sc = mla_store_partial<F16>(p.part_o + prow * 512 + DPW * w + 4 * EPL * g, ov, inv);
+  if (F16 && g == 0) {
+#pragma unroll
+    for (int i = 0; i < DPW / 64; ++i) p.part_sc[prow * 8 + (DPW / 64) * w + i] = sc;
   }
   if (w == 0 && g == 0) *reinterpret_cast<float2 *>(p.part_ml + prow * 2) = make_float2(acc.m, l_tot);
 }
@@ -1271,7 +1508,17 @@ __device__ __forceinline__ void mla_attention_body(const MlaParams &p, const Mla
   using Cfg = MlaCfg<F, SPARSE, WIDE>;
   constexpr int NW = Cfg::NW;
   __shared__ __align__(16) uint8_t ring[Cfg::RING];
-  __shared__ __align__(16) float xbuf[Cfg::XB * NW * 64][8];  // score exchange
+  __shared__ __align__(16) float xbuf_own[Cfg::XBUF > 0 ? Cfg::XBUF : 1][8];  // score exchange
+  float (*xbuf)[8] = Cfg::XBUF > 0 ? xbuf_own : reinterpret_cast<float (*)[8]>(&ring[0]);
+  float (*s_max)[16] = nullptr;  // the row-quantized layout's maxima and flag
+  int *s_over = nullptr;
+  if constexpr (Cfg::RQ) {
+    __shared__ float rq_max[NW][16];
+    __shared__ int rq_over;
+    s_max = rq_max;
+    s_over = &rq_over;
+    if (threadIdx.x == 0) rq_over = 0;
+  }
   // The sparse slot list lives in the workgroup's LDS only for sparse calls
   // (the dense C8 variant fits two workgroups per CU exactly).
   uint32_t *slot_list = nullptr;
@@ -1383,7 +1630,7 @@ __device__ __forceinline__ void mla_attention_body(const MlaParams &p, const Mla
       const int slot0 =
           self ? mla_se_slot(s_se[row]) : (gplan ? p.row_slot[row].x : ld_const(&p.row_slot[row].x));
       if (sinks && mla_sink_mid(p, pos) >= lo && mla_sink_mid(p, pos) < hi) {
-        mla_sink_item<NW, Cfg::WGS == 1>(p, xbuf, row, slot0, w, lane);
+        mla_sink_item<NW, Cfg::WGS == 1, Cfg::RQ>(p, xbuf, row, slot0, w, lane);
         __syncthreads();  // every wave is done with xbuf
       }
       const int seq = !p.cu_q ? row : (self || gplan ? mla_seq_of(p, row) : ld_const(p.row_seq + row));
@@ -1396,7 +1643,10 @@ __device__ __forceinline__ void mla_attention_body(const MlaParams &p, const Mla
       j1 = uniform(j1 < rw.tiles ? j1 : rw.tiles);
       if (j0 >= j1) continue;
       const int slot = uniform(slot0 >= 0 ? slot0 + sinks + (v - rw.wa) : -1);
-      mla_item<F, SPARSE, WIDE>(p, ring, xbuf, slot_list, row, sp, j0, j1, slot, w, lane);
+      if constexpr (Cfg::RQ)
+        mla_rq_item<F>(p, ring, s_max, s_over, row, sp, j0, j1, slot, w, lane);
+      else
+        mla_item<F, SPARSE, WIDE>(p, ring, xbuf, slot_list, row, sp, j0, j1, slot, w, lane);
       __syncthreads();  // every wave is done with xbuf (and the ring)
     }
   }
@@ -1413,74 +1663,123 @@ __global__ __launch_bounds__(64 * (MlaCfg<F, false, WIDE>::NW), (MlaCfg<F, false
 }
 
 // Combine one (row, head): the row's partials (the sink partial first, when
-// there are sinks, then one per share its tiles touch). Each thread owns 2
-// output dims.
+// there are sinks, then one per share its tiles touch). Bound by round trips,
+// not bytes, so all of them are loaded at once. Up to kFast partials: every
+// thread loads its two dims and (m, l) of each. More: wave u takes partials u,
+// u + 4, ... (lane l dims 8l .. 8l + 7, up to kBatch 16-byte loads in flight, those
+// past the last partial out of the buffer's range), every wave reads all (m, l)
+// (lane k: partial k) and takes the weights from them, and the waves' sums meet in
+// LDS (a C8 step of 128 rows over 1024..65536 keys, up to 40 partials a row:
+// 268.6 -> 267.4 us; taken for few partials too it cost the window call 1.3 us).
+template <bool F16>
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
-  const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
+  auto pair = [](uint32_t word) {  // two dims of a partial
+    if constexpr (F16) {
+      const f16x2 x = __builtin_bit_cast(f16x2, word);
+      return f32x2{float(x[0]), float(x[1])};
+    } else {
+      return f32x2{bf16_bits_to_f32(word & 0xFFFFu), bf16_bits_to_f32(word >> 16)};
+    }
+  };
+  constexpr int kBatch = 8, kFast = 8;
+  const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int wv = uniform(tid >> 6);
   const int2 slots = make_int2(ld_const(&p.row_slot[row].x), ld_const(&p.row_slot[row].y));
   if (slots.x < 0) return;  // output written by the attention kernel or the plan
-  const int slot0 = slots.x, total = slots.y;
-  const int64_t prow0 = int64_t(slot0) * p.heads + h;
-  auto part_at = [&](int k) { return prow0 + int64_t(k) * p.heads; };
+  const int total = slots.y;
+  const int64_t prow0 = int64_t(slots.x) * p.heads + h;
   uint32_t *op = reinterpret_cast<uint32_t *>(p.out + (int64_t(row) * p.heads + h) * 512) + tid;
-  constexpr int kFast = 8;
   if (total <= kFast) {
-    // One round trip: every (m, l) and O word of the row's partials is loaded
-    // together (indices past the last partial repeat it with weight 0) and
-    // each thread takes the max itself.
-    float2 m_l[kFast];
+    float2 ml[kFast];
+    float sc[kFast];
     uint32_t o[kFast];
 #pragma unroll
-    for (int k = 0; k < kFast; ++k) {
-      const int64_t pr = part_at(k < total ? k : total - 1);
-      m_l[k] = *reinterpret_cast<const float2 *>(p.part_ml + pr * 2);
-      o[k] = *reinterpret_cast<const uint32_t *>(p.part_o + pr * 512 + 2 * tid);
+    for (int k = 0; k < kFast; ++k) {  // indices past the last partial repeat it with weight 0
+      const int64_t r = prow0 + int64_t(k < total ? k : total - 1) * p.heads;
+      ml[k] = *reinterpret_cast<const float2 *>(p.part_ml + r * 2);
+      sc[k] = F16 ? p.part_sc[r * 8 + (tid >> 5)] : 1.0f;
+      o[k] = *reinterpret_cast<const uint32_t *>(p.part_o + r * 512 + 2 * tid);
     }
-    float Mt = -INFINITY;
+    float mx = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < kFast; ++k) Mt = fmaxf(Mt, m_l[k].x);
-    if (Mt == -INFINITY) {  // nothing visible
+    for (int k = 0; k < kFast; ++k) mx = fmaxf(mx, ml[k].x);
+    if (mx == -INFINITY) {  // nothing visible
       *op = 0u;
       return;
     }
-    float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
+    float l = 0.0f, o0 = 0.0f, o1 = 0.0f;
 #pragma unroll
-    for (int k = 0; k < kFast; ++k) {
-      const float wk = k < total ? fast_exp2(m_l[k].x - Mt) * m_l[k].y : 0.0f;  // partials hold O / l
-      L += wk;
-      o0 += wk * bf16_bits_to_f32(o[k] & 0xFFFFu);
-      o1 += wk * bf16_bits_to_f32(o[k] >> 16);
+    for (int k = 0; k < kFast; ++k) {  // partials hold O / l
+      const float wk = k < total ? fast_exp2(ml[k].x - mx) * ml[k].y : 0.0f;
+      const f32x2 x = pair(o[k]);
+      l += wk;
+      const float f = F16 ? wk * sc[k] : wk;
+      o0 += f * x[0];
+      o1 += f * x[1];
     }
-    const float inv = 1.0f / L;
+    const float inv = 1.0f / l;
     *op = pack_bf16x2(o0 * inv, o1 * inv);
     return;
   }
-  // Largest partial max: threads stride over the partials, then a
-  // workgroup reduction (4 waves).
-  __shared__ float wmax[4];
-  float mp = -INFINITY;
-  for (int k = tid; k < total; k += 256) mp = fmaxf(mp, p.part_ml[part_at(k) * 2]);
+  __shared__ float s_acc[4][512];
+  const uint32_t stride = uint32_t(p.heads), rows = uint32_t(total) * stride;
+  const auto ro = make_rsrc(p.part_o + prow0 * 512, rows * 1024u);
+  const auto rs = make_rsrc(p.part_sc + prow0 * 8, rows * 32u);
+  const auto rm = make_rsrc(p.part_ml + prow0 * 2, rows * 8u);
+  u32x4 o[kBatch];
+  float sc[kBatch];
+  auto load = [&](int k0) {
 #pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) mp = wave_max_xor(mp, m);
-  if ((tid & 63) == 0) wmax[tid >> 6] = mp;
-  __syncthreads();
-  const float Mt = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-  if (Mt == -INFINITY) {  // nothing visible
+    for (int u = 0; u < kBatch; ++u) {
+      const uint32_t r = uint32_t(k0 + wv + 4 * u) * stride;
+      o[u] = buf_load_x4(ro, r * 1024u + 16u * uint32_t(lane));
+      sc[u] = F16 ? buf_load_f32(rs, r * 32u + 4u * uint32_t(lane >> 3)) : 1.0f;
+    }
+  };
+  load(0);
+  // (m, l) of partial k + lane, and the largest m of all partials.
+  auto load_ml = [&](int k) {
+    const uint32_t off = uint32_t(k + lane) * stride * 8u;
+    return make_float2(k + lane < total ? buf_load_f32(rm, off) : -INFINITY, buf_load_f32(rm, off + 4));
+  };
+  float2 ml = load_ml(0);
+  float mx = ml.x;
+  for (int k = 64; k < total; k += 64) mx = fmaxf(mx, load_ml(k).x);
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) mx = wave_max_xor(mx, m);
+  if (mx == -INFINITY) {  // nothing visible
     *op = 0u;
     return;
   }
-  float L = 0.0f, o0 = 0.0f, o1 = 0.0f;
-#pragma unroll 8
-  for (int k = 0; k < total; ++k) {
-    const int64_t pr = part_at(k);
-    const float2 m_l = *reinterpret_cast<const float2 *>(p.part_ml + pr * 2);
-    const uint32_t o = *reinterpret_cast<const uint32_t *>(p.part_o + pr * 512 + 2 * tid);
-    const float wk = fast_exp2(m_l.x - Mt) * m_l.y;  // partials hold O / l
-    L += wk;
-    o0 += wk * bf16_bits_to_f32(o & 0xFFFFu);
-    o1 += wk * bf16_bits_to_f32(o >> 16);
+  float l = 0.0f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int k0 = 0; k0 < total; k0 += 4 * kBatch) {
+    if (k0 > 0) load(k0);
+    if (k0 > 0 && (k0 & 63) == 0) ml = load_ml(k0);
+    const float w = fast_exp2(ml.x - mx) * ml.y;  // partials hold O / l
+    if ((k0 & 63) == 0) l += w;
+#pragma unroll
+    for (int u = 0; u < kBatch; ++u) {
+      const float wk = __shfl(w, (k0 & 63) + wv + 4 * u, 64), f = F16 ? wk * sc[u] : wk;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const f32x2 x = pair(o[u][e]);
+        acc[2 * e] += f * x[0];
+        acc[2 * e + 1] += f * x[1];
+      }
+    }
   }
-  const float inv = 1.0f / L;
+#pragma unroll
+  for (int m = 32; m >= 1; m >>= 1) l = wave_sum_xor(l, m);
+  *reinterpret_cast<f32x4 *>(&s_acc[wv][8 * lane]) = f32x4{acc[0], acc[1], acc[2], acc[3]};
+  *reinterpret_cast<f32x4 *>(&s_acc[wv][8 * lane + 4]) = f32x4{acc[4], acc[5], acc[6], acc[7]};
+  __syncthreads();
+  float o0 = 0.0f, o1 = 0.0f;
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    o0 += s_acc[u][2 * tid];
+    o1 += s_acc[u][2 * tid + 1];
+  }
+  const float inv = 1.0f / l;
   *op = pack_bf16x2(o0 * inv, o1 * inv);
 }
 
@@ -1537,11 +1836,9 @@ inline int mla_skew_pm(bool c8, bool sparse, bool wide, bool sinks) {
 // tiles (C8, row-quantized), measured on config-5 rows against equal shares
 // on the same box: C8 0.334-0.335 -> 0.320-0.326 ms at 1400/1000/600
 // (1100/1000/900 and 1300/1000/700 gained less; 1500/1000/500 and
-// 1600/1000/400 measured 0.334-0.343 against 0.328 ms on a later box), int4
-// rows 0.435-0.439 -> 0.399-0.402 ms at 1400/1000/600, and 0.409-0.411 ->
-// 0.400-0.402 ms from 1400/1000/600 to 1500/1000/500 on the later box; int8
-// rows (two per CU) 0.480-0.503 -> 0.464-0.470 ms at 1300/1000, and
-// 0.469-0.479 -> 0.467-0.468 ms at 1500/1000 on the later box. Sparse calls (two per CU) were 2-6% slower
+// 1600/1000/400 measured 0.334-0.343 against 0.328 ms on a later box);
+// row-quantized rows (two per CU) at 1500/1000 int8 0.2705 -> 0.262 and int4
+// 0.326 -> 0.303 ms (1200/1000: 0.267 and 0.3135 ms). Sparse calls (two per CU) were 2-6% slower
 // with weights and keep equal shares; the wide bf16 variant (no LDS for the
 // table) always does.
 // IFATTN_MLA_SLOT_WEIGHTS ("w0,w1[,w2]") overrides the weights of every
@@ -1570,8 +1867,7 @@ inline void mla_slot_weights(MlaParams &p, int wgs, int fmt, bool sparse, bool w
   else if (fmt == kFmtC8)
     w = std::array<int, kMlaSlotsMax>{1400, 1000, 600};
   else
-    w = wgs == 3 ? std::array<int, kMlaSlotsMax>{1500, 1000, 500}
-                 : std::array<int, kMlaSlotsMax>{1500, 1000, 0};
+    w = std::array<int, kMlaSlotsMax>{1500, 1000, 0};
   // Malformed weights: equal shares.
   int wsum = 0;
   for (int k = 0; k < wgs; ++k) wsum += w[k];
@@ -1620,7 +1916,7 @@ inline uint64_t mla_workspace(int rows, int heads, bool sparse, int topk, int n_
   const uint64_t workers = mla_max_workers(sparse, rows, topk, n_sinks);
   const uint64_t slots = mla_slots(workers, rows, n_sinks);
   return kQueueBytes + 2 * align16(uint64_t(rows) * 8) + align16(uint64_t(rows) * 4) +
-         align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 2 * sizeof(float));
+         align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 10 * sizeof(float));
 }
 
 int32_t mla_run(const MlaCall &c, const char *what) {
@@ -1724,7 +2020,8 @@ int32_t mla_run(const MlaCall &c, const char *what) {
   ws += align16(max_workers * 4);
   const uint64_t slots = mla_slots(max_workers, c.num_rows, c.n_sinks);
   p.part_o = reinterpret_cast<uint16_t *>(ws);
-  p.part_ml = reinterpret_cast<float *>(p.part_o + slots * c.heads * 512);
+  p.part_sc = reinterpret_cast<float *>(p.part_o + slots * c.heads * 512);
+  p.part_ml = p.part_sc + slots * c.heads * 8;
   hipStream_t s = static_cast<hipStream_t>(c.stream);
   if (!p.self_plan) mla_plan_kernel<<<1, 1024, 0, s>>>(p);
   constexpr int kThreads = 64 * kMlaWaves;
@@ -1748,7 +2045,8 @@ int32_t mla_run(const MlaCall &c, const char *what) {
     else if (step) mla_step_kernel<kFmtBf16, false><<<grid, kThreads, 0, s>>>(p, st);
     else mla_attention_kernel<kFmtBf16, false, false><<<grid, kThreads, 0, s>>>(p);
   }
-  mla_merge_kernel<<<dim3(c.num_rows, c.heads), 256, 0, s>>>(p);
+  if (rq) mla_merge_kernel<true><<<dim3(c.num_rows, c.heads), 256, 0, s>>>(p);
+  else mla_merge_kernel<false><<<dim3(c.num_rows, c.heads), 256, 0, s>>>(p);
   return launch_status(what);
 }
 

@@ -186,3 +186,37 @@ def test_state_allocation_failure_cleans_up(monkeypatch):
     assert all(b[k] for k in ("cache", "table", "scales", "query", "out", "indices", "kv_len",
                               "sink_keys", "sink_values"))
     assert os.environ.get("IFATTN_STATE_FAIL_ALLOCATION") is None
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+def test_rowq_step_edges(bits):
+    # lengths around the wave (16 keys), step (64 keys) and buffer (128 keys) edges
+    kv = [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129, 191, 193, 640]
+    q, packed, scales, deq, table, kv, _, maxc = batch(31, [1] * len(kv), kv, 16, 6, bits)
+    for window in (0, 20, 100):
+        got = run(q, packed, scales, bits, table, kv, maxc, window=window)
+        exp = oracle.mla_attention(q, deq, table, kv, 6, 16, SCALE, window=window)
+        assert_close(got, exp)
+
+
+@pytest.mark.parametrize("bits", [8, 4])
+@pytest.mark.parametrize("at", [70, 150, 290])
+def test_rowq_scores_jump_beyond_the_running_max(bits, at):
+    # From position `at` on, keys whose scores exceed all earlier ones by more
+    # than 2^64: the step that meets them takes a new base before P is used
+    # (and a later, smaller jump moves it after PV).
+    q, packed, scales, deq, table, kv, _, maxc = batch(33, [1], [300], 16, 6, bits)
+    rng = np.random.default_rng(34)
+    d = rng.choice([-1.0, 1.0], 576).astype(f32)
+    q[0] = bf(np.tile(d, (6, 1)) * f32(1.5))
+    pool = packed.reshape(-1, packed.shape[2])
+    pos = np.arange(at, 300)
+    slots = table[0, pos // 16].astype(np.int64) * 16 + pos % 16
+    rows = bf(d[None] * (2.0 + 0.01 * np.arange(pos.size))[:, None].astype(f32)
+              + rng.standard_normal((pos.size, 576)).astype(f32) * f32(0.5))
+    pool[slots], scales[slots], deq[slots] = quantize_pool(rows, bits)
+    got = run(q, packed, scales, bits, table, kv, maxc)
+    exp = oracle.mla_attention(q, deq, table, kv, 6, 16, SCALE)
+    x = (W.bf16_to_f32(q[0, 0]) @ W.bf16_to_f32(deq[slots[0]])) * SCALE * 1.4427
+    assert x > 80
+    assert_close(got, exp)
