@@ -81,9 +81,8 @@ struct MlaParams {
   int2 *row_slot;               // [rows] (first partial slot, slot count); (-1, 0): the row
                                 // writes its output directly
   int32_t *start_row;           // [max_workers] first row not wholly before each worker's share
-  uint16_t *part_o;             // [slots, heads, 512] O / l of each partial: bf16, or scaled fp16
-  float *part_sc;               // [slots, heads, 8] inverse scale of each 64 dims (fp16 partials)
-  float *part_ml;               // [slots, heads, 2]
+  uint16_t *part_o;             // [slots, heads, 512] scaled fp16 O / l of each partial
+  float *part_ml;               // [slots, heads, 8] m, l, two unused, inverse scale of each 128 dims
   int64_t num_blocks;
   uint32_t cache_bytes;  // sparse and row-quantized gathers: byte extent of the cache (< 4 GiB - 16)
   uint32_t scale_bytes;  // row-quantized rows: byte extent of row_scales
@@ -260,12 +259,11 @@ __device__ __forceinline__ int64_t mla_row_weight(const MlaParams &p, const MlaS
   const int tiles = mla_tiles(sp);
   return (tiles > 0 ? int64_t(p.row_cost) + int64_t(kMlaTile) * tiles : 0) + p.sink_units;
 }
-// Workers of a call of `total` units: the grid, fewer for small calls (at
-// least kMinShareUnits each), more for sparse calls whose shares must fit the
-// slot list, at most the workspace's max_workers.
+// Workers of a call of `total` units: the grid, fewer for small calls
+// (split_workers), more for sparse calls whose shares must fit the slot list, at
+// most the workspace's max_workers.
 __device__ __forceinline__ int mla_split(const MlaParams &p, int64_t total) {
-  const int64_t small = (total + kMinShareUnits - 1) / kMinShareUnits;
-  int64_t wk = small < p.grid ? small : p.grid;
+  int64_t wk = split_workers(total, 1, p.slot_c, p.grid);
   const int64_t bound = (total + p.max_share - 1) / p.max_share;  // sparse share cap
   wk = bound > wk ? bound : wk;
   wk = wk < 1 ? 1 : (wk > p.max_workers ? p.max_workers : wk);
@@ -503,36 +501,32 @@ struct MlaGeo {
 
 constexpr uint32_t kNoRow = 0xFFFFFFFFu;  // sparse slot list: no key
 
-// A lane's N consecutive dims of a partial's O / l (o times inv). Row-quantized
-// rows (F16) hold them in fp16 under a power-of-two scale over the four lanes (g)
-// that share the wave's dims: the bytes of bf16 with 2^-11 of the largest value
-// as the worst rounding instead of 2^-8 of each, which their large rows need to
-// stay within the outputs' bound (a split of the call into other shares moved
-// one past it). The other formats hold bf16 (the scale costs the small window
-// and sparse calls 1-3%). Returns the inverse scale.
-template <bool F16, int N>
-__device__ __forceinline__ float mla_store_partial(uint16_t *po, const float (&o)[N], float inv) {
-  if constexpr (!F16) {
-#pragma unroll
-    for (int k = 0; k < N; k += 8)
-      store_u32x4(po + k, u32x4{pack_bf16x2(o[k] * inv, o[k + 1] * inv),
-                                pack_bf16x2(o[k + 2] * inv, o[k + 3] * inv),
-                                pack_bf16x2(o[k + 4] * inv, o[k + 5] * inv),
-                                pack_bf16x2(o[k + 6] * inv, o[k + 7] * inv)});
-    return 1.0f;
-  }
+// Partials hold O / l in fp16 under a power-of-two scale of each head and 128
+// dims: the bytes of bf16 with 2^-11 of the largest value as the worst rounding
+// instead of 2^-8 of each, so that cutting a row into more shares costs no
+// precision (error against 64 bits of a window-2048 call 0.0026 with bf16
+// partials, 0.0021). Stores a lane's 32 consecutive dims (o times inv), scaled
+// over the four lanes (g) that share the wave's 128, to partial row prow, and
+// the wave's entry of its (m, l, scales).
+__device__ __forceinline__ void mla_store_partial(const MlaParams &p, int64_t prow, int w, int g,
+                                                  const float (&o)[32], float inv, float m, float l) {
   float amax = 0.0f;
 #pragma unroll
-  for (int i = 0; i < N; ++i) amax = fmaxf(amax, fabsf(o[i]));
+  for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(o[i]));
   const float ps = f16_range_scale(max_xor32(max_xor16(amax * inv)));
   const float f = inv * ps;
+  uint16_t *po = p.part_o + prow * 512 + 128 * w + 32 * g;
   auto two = [&](int i) {
     const f16x2 h = __builtin_convertvector((f32x2{o[i] * f, o[i + 1] * f}), f16x2);
     return __builtin_bit_cast(uint32_t, h);
   };
 #pragma unroll
-  for (int k = 0; k < N; k += 8) store_u32x4(po + k, u32x4{two(k), two(k + 2), two(k + 4), two(k + 6)});
-  return __uint_as_float((254u << 23) - __float_as_uint(ps));  // 1 / ps
+  for (int k = 0; k < 32; k += 8) store_u32x4(po + k, u32x4{two(k), two(k + 2), two(k + 4), two(k + 6)});
+  if (g == 0) {
+    float *e = p.part_ml + prow * 8;
+    e[4 + w] = __uint_as_float((254u << 23) - __float_as_uint(ps));  // 1 / ps
+    if (w == 0) *reinterpret_cast<float2 *>(e) = make_float2(m, l);
+  }
 }
 
 __device__ __forceinline__ int mla_tile_token(int g, int j) {
@@ -1005,8 +999,8 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
   } else {
     const int64_t prow = int64_t(slot) * p.heads + c;
     const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    mla_store_partial<false>(p.part_o + prow * DV + d0, ov, inv);
-    if (w == 0 && g == 0) *reinterpret_cast<float2 *>(p.part_ml + prow * 2) = make_float2(acc.m, l_tot);
+    static_assert(DPW == 128, "one scale entry per wave");
+    mla_store_partial(p, prow, w, g, ov, inv, acc.m, l_tot);
   }
 }
 
@@ -1264,9 +1258,7 @@ __device__ __forceinline__ void mla_rq_item(const MlaParams &p, uint8_t *ring, f
                                 pack_bf16x2(ov[k + 6] * inv, ov[k + 7] * inv)});
   } else {
     const int64_t prow = int64_t(slot) * p.heads + c;
-    const float sc = mla_store_partial<true>(p.part_o + prow * 512 + 128 * w + 32 * g, ov, inv);
-    if (g == 0) *reinterpret_cast<float2 *>(p.part_sc + prow * 8 + 2 * w) = make_float2(sc, sc);
-    if (w == 0 && g == 0) *reinterpret_cast<float2 *>(p.part_ml + prow * 2) = make_float2(m_run, l_tot);
+    mla_store_partial(p, prow, w, g, ov, inv, m_run, l_tot);
   }
 }
 
@@ -1275,7 +1267,7 @@ __device__ __forceinline__ void mla_rq_item(const MlaParams &p, uint8_t *ring, f
 // cache keys, four waves per row, heads in the MFMA N dimension. The (m, l, O)
 // partial of the sinks alone goes to the row's first partial slot. Runs as the
 // event at the start of the row's work units, in the share that holds it.
-template <int NW, bool DB, bool F16>
+template <int NW, bool DB>
 __device__ __forceinline__ void mla_sink_item(const MlaParams &p, float (*xbuf)[8], int row, int slot0,
                                               int w, int lane) {
   using Geo = MlaGeo<NW>;
@@ -1356,12 +1348,7 @@ __device__ __forceinline__ void mla_sink_item(const MlaParams &p, float (*xbuf)[
   for (int r = 0; r < 4; ++r)
 #pragma unroll
     for (int b = 0; b < EPL; ++b) ov[EPL * r + b] = acc.o[b][r];
-  const float sc = mla_store_partial<F16>(p.part_o + prow * 512 + DPW * w + 4 * EPL * g, ov, inv);
-  if (F16 && g == 0) {
-#pragma unroll
-    for (int i = 0; i < DPW / 64; ++i) p.part_sc[prow * 8 + (DPW / 64) * w + i] = sc;
-  }
-  if (w == 0 && g == 0) *reinterpret_cast<float2 *>(p.part_ml + prow * 2) = make_float2(acc.m, l_tot);
+  mla_store_partial(p, prow, w, g, ov, inv, acc.m, l_tot);
 }
 
 // Rows a workgroup plans for itself (one per thread): calls of at most this
@@ -1630,7 +1617,7 @@ __device__ __forceinline__ void mla_attention_body(const MlaParams &p, const Mla
       const int slot0 =
           self ? mla_se_slot(s_se[row]) : (gplan ? p.row_slot[row].x : ld_const(&p.row_slot[row].x));
       if (sinks && mla_sink_mid(p, pos) >= lo && mla_sink_mid(p, pos) < hi) {
-        mla_sink_item<NW, Cfg::WGS == 1, Cfg::RQ>(p, xbuf, row, slot0, w, lane);
+        mla_sink_item<NW, Cfg::WGS == 1>(p, xbuf, row, slot0, w, lane);
         __syncthreads();  // every wave is done with xbuf
       }
       const int seq = !p.cu_q ? row : (self || gplan ? mla_seq_of(p, row) : ld_const(p.row_seq + row));
@@ -1671,16 +1658,8 @@ __global__ __launch_bounds__(64 * (MlaCfg<F, false, WIDE>::NW), (MlaCfg<F, false
 // (lane k: partial k) and takes the weights from them, and the waves' sums meet in
 // LDS (a C8 step of 128 rows over 1024..65536 keys, up to 40 partials a row:
 // 268.6 -> 267.4 us; taken for few partials too it cost the window call 1.3 us).
-template <bool F16>
 __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
-  auto pair = [](uint32_t word) {  // two dims of a partial
-    if constexpr (F16) {
-      const f16x2 x = __builtin_bit_cast(f16x2, word);
-      return f32x2{float(x[0]), float(x[1])};
-    } else {
-      return f32x2{bf16_bits_to_f32(word & 0xFFFFu), bf16_bits_to_f32(word >> 16)};
-    }
-  };
+  auto pair = [](uint32_t word) { return __builtin_bit_cast(f16x2, word); };  // two dims of a partial
   constexpr int kBatch = 8, kFast = 8;
   const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int wv = uniform(tid >> 6);
@@ -1696,8 +1675,9 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
 #pragma unroll
     for (int k = 0; k < kFast; ++k) {  // indices past the last partial repeat it with weight 0
       const int64_t r = prow0 + int64_t(k < total ? k : total - 1) * p.heads;
-      ml[k] = *reinterpret_cast<const float2 *>(p.part_ml + r * 2);
-      sc[k] = F16 ? p.part_sc[r * 8 + (tid >> 5)] : 1.0f;
+      const float *e = p.part_ml + r * 8;  // wave-uniform: scalar loads
+      ml[k] = make_float2(ld_const(e), ld_const(e + 1));
+      sc[k] = ld_const(e + 4 + wv);
       o[k] = *reinterpret_cast<const uint32_t *>(p.part_o + r * 512 + 2 * tid);
     }
     float mx = -INFINITY;
@@ -1711,11 +1691,11 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
 #pragma unroll
     for (int k = 0; k < kFast; ++k) {  // partials hold O / l
       const float wk = k < total ? fast_exp2(ml[k].x - mx) * ml[k].y : 0.0f;
-      const f32x2 x = pair(o[k]);
+      const f16x2 x = pair(o[k]);
       l += wk;
-      const float f = F16 ? wk * sc[k] : wk;
-      o0 += f * x[0];
-      o1 += f * x[1];
+      const float f = wk * sc[k];
+      o0 += f * float(x[0]);
+      o1 += f * float(x[1]);
     }
     const float inv = 1.0f / l;
     *op = pack_bf16x2(o0 * inv, o1 * inv);
@@ -1724,8 +1704,7 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
   __shared__ float s_acc[4][512];
   const uint32_t stride = uint32_t(p.heads), rows = uint32_t(total) * stride;
   const auto ro = make_rsrc(p.part_o + prow0 * 512, rows * 1024u);
-  const auto rs = make_rsrc(p.part_sc + prow0 * 8, rows * 32u);
-  const auto rm = make_rsrc(p.part_ml + prow0 * 2, rows * 8u);
+  const auto rm = make_rsrc(p.part_ml + prow0 * 8, rows * 32u);
   u32x4 o[kBatch];
   float sc[kBatch];
   auto load = [&](int k0) {
@@ -1733,13 +1712,13 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
     for (int u = 0; u < kBatch; ++u) {
       const uint32_t r = uint32_t(k0 + wv + 4 * u) * stride;
       o[u] = buf_load_x4(ro, r * 1024u + 16u * uint32_t(lane));
-      sc[u] = F16 ? buf_load_f32(rs, r * 32u + 4u * uint32_t(lane >> 3)) : 1.0f;
+      sc[u] = buf_load_f32(rm, r * 32u + 16u + 4u * uint32_t(lane >> 4));
     }
   };
   load(0);
   // (m, l) of partial k + lane, and the largest m of all partials.
   auto load_ml = [&](int k) {
-    const uint32_t off = uint32_t(k + lane) * stride * 8u;
+    const uint32_t off = uint32_t(k + lane) * stride * 32u;
     return make_float2(k + lane < total ? buf_load_f32(rm, off) : -INFINITY, buf_load_f32(rm, off + 4));
   };
   float2 ml = load_ml(0);
@@ -1759,12 +1738,12 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
     if ((k0 & 63) == 0) l += w;
 #pragma unroll
     for (int u = 0; u < kBatch; ++u) {
-      const float wk = __shfl(w, (k0 & 63) + wv + 4 * u, 64), f = F16 ? wk * sc[u] : wk;
+      const float wk = __shfl(w, (k0 & 63) + wv + 4 * u, 64), f = wk * sc[u];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const f32x2 x = pair(o[u][e]);
-        acc[2 * e] += f * x[0];
-        acc[2 * e + 1] += f * x[1];
+        const f16x2 x = pair(o[u][e]);
+        acc[2 * e] += f * float(x[0]);
+        acc[2 * e + 1] += f * float(x[1]);
       }
     }
   }
@@ -1916,7 +1895,7 @@ inline uint64_t mla_workspace(int rows, int heads, bool sparse, int topk, int n_
   const uint64_t workers = mla_max_workers(sparse, rows, topk, n_sinks);
   const uint64_t slots = mla_slots(workers, rows, n_sinks);
   return kQueueBytes + 2 * align16(uint64_t(rows) * 8) + align16(uint64_t(rows) * 4) +
-         align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 10 * sizeof(float));
+         align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 8 * sizeof(float));
 }
 
 int32_t mla_run(const MlaCall &c, const char *what) {
@@ -2020,8 +1999,7 @@ int32_t mla_run(const MlaCall &c, const char *what) {
   ws += align16(max_workers * 4);
   const uint64_t slots = mla_slots(max_workers, c.num_rows, c.n_sinks);
   p.part_o = reinterpret_cast<uint16_t *>(ws);
-  p.part_sc = reinterpret_cast<float *>(p.part_o + slots * c.heads * 512);
-  p.part_ml = p.part_sc + slots * c.heads * 8;
+  p.part_ml = reinterpret_cast<float *>(p.part_o + slots * c.heads * 512);
   hipStream_t s = static_cast<hipStream_t>(c.stream);
   if (!p.self_plan) mla_plan_kernel<<<1, 1024, 0, s>>>(p);
   constexpr int kThreads = 64 * kMlaWaves;
@@ -2045,8 +2023,7 @@ int32_t mla_run(const MlaCall &c, const char *what) {
     else if (step) mla_step_kernel<kFmtBf16, false><<<grid, kThreads, 0, s>>>(p, st);
     else mla_attention_kernel<kFmtBf16, false, false><<<grid, kThreads, 0, s>>>(p);
   }
-  if (rq) mla_merge_kernel<true><<<dim3(c.num_rows, c.heads), 256, 0, s>>>(p);
-  else mla_merge_kernel<false><<<dim3(c.num_rows, c.heads), 256, 0, s>>>(p);
+  mla_merge_kernel<<<dim3(c.num_rows, c.heads), 256, 0, s>>>(p);
   return launch_status(what);
 }
 

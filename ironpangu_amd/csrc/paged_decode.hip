@@ -593,9 +593,7 @@ __device__ __forceinline__ void decode_self_plan_wg(const DecodeParams &p, int *
   int total;
   const int pos0 = decode_wg_scan<false>(sum, s_wt, &total);
   {
-    const int64_t small = (int64_t(total) + kMinShareUnits - 1) / kMinShareUnits;
-    workers = int(small < p.grid ? small : p.grid);
-    workers = workers < 1 ? 1 : workers;
+    workers = int(split_workers(total, p.groups, p.cus, p.grid));
     share = total > 0 ? (int64_t(total) + workers - 1) / workers : 1;
   }
   int cnt[K], last[K], csum = 0, emine = -1;
@@ -692,6 +690,7 @@ void launch_decode(const DecodeParams &p0, const RowWrite &wr, hipStream_t s) {
   const int waves = p0.kv_heads < max_decode_waves(D) ? p0.kv_heads : max_decode_waves(D);
   DecodeParams p = p0;
   p.seq_cost = decode_seq_cost(C8);
+  p.groups = (p.kv_heads + waves - 1) / waves;
   p.self_plan = decode_self_plan(p, 64 * waves) ? 1 : 0;
   p.skew_pm = decode_skew_pm(C8, D);
   launch_prologue(p, wr, s);

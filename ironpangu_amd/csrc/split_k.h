@@ -49,6 +49,7 @@ struct DecodeParams {
   int num_seqs, q_heads, kv_heads, group, table_stride, block_size, max_context, head_dim;
   int seq_cost;      // work units charged per sequence on top of its tokens
   int grid;          // persistent decode workgroups (the most workers)
+  int cus, groups;   // compute units; passes over the kv heads per tile (split_workers)
   int self_plan;     // the decode workgroups plan the call themselves (prologue: row writes only)
   int skew_pm;       // share skew d = S * skew_pm / 1000 (see Shares)
   float scale_log2;  // softmax scale * log2(e)
@@ -149,9 +150,28 @@ __device__ __forceinline__ void prologue_write(const RowWrite &w) {
   }
 }
 
-// Smallest share the plan cuts (units): tiny calls use fewer workers instead of
-// spreading every sequence over many one-tile shares.
-constexpr int64_t kMinShareUnits = 512;
+// Workers of a call of `total` units (each costing `groups` passes over the kv
+// heads), at most `grid`. A call that cannot fill one workgroup per CU is cut into
+// shares of kMinShareUnits: its time is the walk of one share plus fixed launch
+// and merge costs, so the walk is made short. Further workgroups on the same CU
+// only pay once each has kFullShareUnits: they add partials and share the CU's
+// bandwidth. Device time per call at 512 units per share -> 96 (with 64 and 128
+// within 1 us of it): 8 bf16 sequences of 16..512 tokens 25.7 -> 16.5 us, 16 int8
+// of 500..3000 28.7 -> 19.7, 4 MLA rows of 200..3000 keys 31.1 -> 16.7, 31
+// row-quantized of 200..360 36.3 -> 18.3; 16 sequences of 500..3000 at head_dim 256
+// 47.3 -> 26.7 us with 227 shares but 32.1 with 302, hence the second line.
+constexpr int64_t kMinShareUnits = 96, kFullShareUnits = 256;
+__device__ __forceinline__ int64_t split_workers(int64_t total, int groups, int cus, int64_t grid) {
+  const int64_t work = total * groups;
+  const int64_t few = (work + kMinShareUnits - 1) / kMinShareUnits;
+  const int64_t full = (work + kFullShareUnits - 1) / kFullShareUnits;
+  const int64_t most = full > cus ? full : cus;
+  int64_t w = few < most ? few : most;
+  const int64_t tiles = (total + kSplitTile - 1) / kSplitTile;
+  w = w < tiles ? w : tiles;
+  w = w < grid ? w : grid;
+  return w < 1 ? 1 : w;
+}
 
 // Workgroup-wide inclusive scan (sum or max) of one value per thread, 1024
 // threads: shuffles within the wave, wave totals through LDS. Returns the
@@ -181,8 +201,7 @@ __device__ __forceinline__ T block_scan(T x, T *wave_tot, T *total) {
 // Pass 1: weights (tokens + seq_cost for a decode sequence with keys, 0
 // otherwise) -> seq_pos by an exclusive scan; sequences without a visible key
 // get their defined zero output here. Then workers = grid, fewer for small
-// calls (at least kMinShareUnits per worker), and share = ceil(total /
-// workers). Pass 2: a
+// calls (split_workers), and share = ceil(total / workers). Pass 2: a
 // sequence whose first and last tiles fall in different shares gets
 // consecutive partial slots (one per share it touches); start_seq[v] = the
 // first sequence whose last tile lies in share v or later.
@@ -223,9 +242,7 @@ __global__ __launch_bounds__(1024) void decode_prologue_kernel(DecodeParams p, R
   }
   if (tid == 0) {
     const long long total = s_pos;
-    const long long small = (total + kMinShareUnits - 1) / kMinShareUnits;
-    long long workers = small < p.grid ? small : p.grid;
-    workers = workers < 1 ? 1 : workers;
+    const long long workers = split_workers(total, p.groups, p.cus, p.grid);
     const long long share = total > 0 ? (total + workers - 1) / workers : 1;
     s_workers = int(workers);
     s_share = share;
@@ -431,6 +448,8 @@ inline uint64_t split_k_workspace_bytes(int num_seqs, int heads, int dims, int /
 inline void split_k_bind_workspace(DecodeParams &p, void *workspace, int heads, int dims) {
   p.seq_cost = decode_seq_cost();
   p.grid = decode_grid();
+  p.cus = device_cus();
+  p.groups = 1;
   p.head_dim = dims;
   uint8_t *w = static_cast<uint8_t *>(workspace);
   p.plan = reinterpret_cast<int32_t *>(w);
