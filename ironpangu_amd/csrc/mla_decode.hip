@@ -263,7 +263,7 @@ __device__ __forceinline__ int64_t mla_row_weight(const MlaParams &p, const MlaS
 // (split_workers), more for sparse calls whose shares must fit the slot list, at
 // most the workspace's max_workers.
 __device__ __forceinline__ int mla_split(const MlaParams &p, int64_t total) {
-  int64_t wk = split_workers(total, 1, p.slot_c, p.grid);
+  int64_t wk = split_workers(total, 1, {256, p.slot_c + p.slot_c / 2}, p.slot_c, p.grid);
   const int64_t bound = (total + p.max_share - 1) / p.max_share;  // sparse share cap
   wk = bound > wk ? bound : wk;
   wk = wk < 1 ? 1 : (wk > p.max_workers ? p.max_workers : wk);

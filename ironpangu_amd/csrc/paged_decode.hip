@@ -593,7 +593,7 @@ __device__ __forceinline__ void decode_self_plan_wg(const DecodeParams &p, int *
   int total;
   const int pos0 = decode_wg_scan<false>(sum, s_wt, &total);
   {
-    workers = int(split_workers(total, p.groups, p.cus, p.grid));
+    workers = int(split_workers(total, p.groups, p.full, p.cus, p.grid));
     share = total > 0 ? (int64_t(total) + workers - 1) / workers : 1;
   }
   int cnt[K], last[K], csum = 0, emine = -1;
@@ -685,12 +685,19 @@ __global__ __launch_bounds__(64 * max_decode_waves(D), 1) void paged_decode_kern
 }
 
 namespace {
+// The classes of FullShares.
+template <int D, bool C8>
+FullShares full_shares(const DecodeParams &p) {
+  if (p.kv_heads < 4 || D == 64) return {256, p.cus + p.cus / 2};
+  return {512, C8 || D > 128 ? p.cus : p.cus / 2 + p.cus / 16};
+}
 template <int D, bool C8>
 void launch_decode(const DecodeParams &p0, const RowWrite &wr, hipStream_t s) {
   const int waves = p0.kv_heads < max_decode_waves(D) ? p0.kv_heads : max_decode_waves(D);
   DecodeParams p = p0;
   p.seq_cost = decode_seq_cost(C8);
   p.groups = (p.kv_heads + waves - 1) / waves;
+  p.full = full_shares<D, C8>(p);
   p.self_plan = decode_self_plan(p, 64 * waves) ? 1 : 0;
   p.skew_pm = decode_skew_pm(C8, D);
   launch_prologue(p, wr, s);
