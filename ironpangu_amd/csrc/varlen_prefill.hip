@@ -27,7 +27,10 @@
 //    overlap one's MFMAs with the other's softmax.
 //  * tiles wholly above the diagonal are never visited; only tiles crossing a
 //    column's limit apply the causal mask.
-//  * query tiles are scheduled longest-first by a device plan kernel.
+//  * query tiles are scheduled longest-first by a device plan kernel;
+//  * calls whose (query tile, kv head) items leave compute units idle (short
+//    prompts, one chunk over a long context) cut the tiles' keys into pieces of
+//    about one CU's share, each leaving a partial for a merge launch.
 #include <cstdlib>
 
 #include "common.h"
@@ -44,8 +47,12 @@ struct PrefillParams {
   const int32_t *cu;
   const int32_t *kv_lens;
   uint16_t *out;
-  uint32_t *items;   // (seq << 12 | query tile), longest first
-  int32_t *n_items;
+  uint2 *items;      // (seq << 12 | query tile, piece word), longest first
+  uint4 *splits;     // the query tiles cut into pieces: (first row, rows, piece word, 0)
+  int32_t *n_items;  // items, splits
+  float *part_o;     // [piece slot, kv head, column, head_dim] O, not yet over l
+  float2 *part_ml;   // [piece slot, kv head, column] m, l
+  int cus;
   int64_t num_blocks;
   int num_seqs, q_heads, kv_heads, group, table_stride, block_size, max_kv, q_tile;
   int max_q_len;   // rows per sequence beyond this are not scheduled (cu_seqlens is device data)
@@ -65,22 +72,46 @@ constexpr int prefill_nb(int d) {  // column blocks per wave
 }
 constexpr int prefill_q_tile(int d, int g) { return kPrefillWaves * prefill_nb(d) * 16 / g; }
 
-// Work list for the multi-row sequences, sorted by the number of key tokens
-// the query tile visits (descending, 256-token buckets).
-__global__ __launch_bounds__(1024) void prefill_plan_kernel(PrefillParams p) {
+// Piece word of an item: piece (10 bits), pieces of its query tile (10 bits), the
+// first partial slot of the tile (12 bits). One piece: no partial.
+__device__ __forceinline__ int piece_of(uint32_t x) { return int(x & 1023u); }
+__device__ __forceinline__ int pieces_of(uint32_t x) { return int((x >> 10) & 1023u); }
+__device__ __forceinline__ int slot_of(uint32_t x) { return int(x >> 20); }
+// ceil(a / b) for 0 <= a < 2^20, 1 <= b: exact, as a + 0.5 is at least 0.5 / b away
+// from every multiple of b.
+__device__ __forceinline__ int ceil_div(int a, int b) {
+  return int((float(a + b - 1) + 0.5f) * __builtin_amdgcn_rcpf(float(b)));
+}
+// A call's tiles are cut only if that shortens its longest walk by at least
+// kMinSavedKeys, and into pieces of at least kMinPieceKeys.
+constexpr int kMinPieceKeys = 256, kMinSavedKeys = 512;
+constexpr int kMaxCutTiles = 1024;
+
+// Work list for the multi-row sequences. Enough items for every CU: sorted by the
+// number of key tokens the query tile visits (descending, 256-token buckets).
+// Fewer (tile, kv head) items than CUs (and the caller launches the merge:
+// may_split): their order does not matter, and the tiles are cut into pieces of
+// at most `most` steps, the smallest of 16 candidates with which the items still
+// fit one per CU.
+__global__ __launch_bounds__(1024) void prefill_plan_kernel(PrefillParams p, int step_keys,
+                                                            bool may_split) {
   constexpr int kBuckets = 1025;
   __shared__ int bucket[kBuckets];
   __shared__ int s_count[1024], s_kv[1024];
+  __shared__ uint2 s_list[kMaxCutTiles];  // (seq << 12 | tile, steps)
+  __shared__ int s_tiles, s_most;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int QT = p.q_tile;
   const int nbk = (p.max_kv + 255) / 256 + 1;  // <= kBuckets (host-checked)
-  for (int b = tid; b < kBuckets; b += 1024) bucket[b] = 0;
-  // Bucket of query tile qt: the key tokens it visits, most work first.
-  auto cost_bucket = [&](int kv, int qt, int count) {
+  if (tid == 0) {
+    s_tiles = 0;
+    s_most = 1 << 30;
+  }
+  // Key tokens that query tile qt visits.
+  auto reach_of = [&](int kv, int qt, int count) {
     const int rows_end = (qt + 1) * QT < count ? (qt + 1) * QT : count;
-    int reach = kv - count + rows_end;
-    reach = reach < 0 ? 0 : (reach > p.max_kv ? p.max_kv : reach);
-    return nbk - 1 - reach / 256;
+    const int reach = kv - count + rows_end;
+    return reach < 0 ? 0 : (reach > p.max_kv ? p.max_kv : reach);
   };
   // Sequences are staged 1024 at a time (one parallel load each); the query
   // tiles of a sequence are then spread over the lanes of one wave, so a long
@@ -100,20 +131,94 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(PrefillParams p) {
       for (int i = wave; i < n; i += 16) {
         const int count = s_count[i];
         if (count <= 1) continue;
-        for (int qt = lane; qt * QT < count; qt += 64) fn(base + i, qt, cost_bucket(s_kv[i], qt, count));
+        for (int qt = lane; qt * QT < count; qt += 64) fn(base + i, qt, reach_of(s_kv[i], qt, count));
       }
     }
   };
-  for_each_tile([&](int, int, int b) { atomicAdd(&bucket[b], 1); });
+  if (may_split) {
+    for_each_tile([&](int seq, int qt, int reach) {
+      const int at = atomicAdd(&s_tiles, 1);
+      if (at < kMaxCutTiles)
+        s_list[at] = make_uint2((uint32_t(seq) << 12) | uint32_t(qt),
+                                uint32_t((reach + step_keys - 1) / step_keys));
+    });
+    __syncthreads();
+    const int tiles = s_tiles, room = p.cus / p.kv_heads;  // items of one kv head
+    if (tiles < room && tiles <= kMaxCutTiles) {
+      int all = 0, longest = 0, sum = 0;
+      for (int t = lane; t < tiles; t += 64) {
+        const int steps = int(s_list[t].y);
+        all += steps;
+        longest = steps > longest ? steps : longest;
+      }
+#pragma unroll
+      for (int m = 32; m >= 1; m >>= 1) {
+        all += __shfl_xor(all, m);
+        const int o = __shfl_xor(longest, m);
+        longest = o > longest ? o : longest;
+      }
+      int least = ceil_div(all, room);
+      least = least * step_keys < kMinPieceKeys ? kMinPieceKeys / step_keys : least;
+      const int most = least + (longest - least) * wave / 16;
+      if ((longest - most) * step_keys >= kMinSavedKeys) {
+        for (int t = lane; t < tiles; t += 64) sum += ceil_div(int(s_list[t].y), most);
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1) sum += __shfl_xor(sum, m);
+        if (lane == 0 && sum <= room) atomicMin(&s_most, most);
+      }
+      __syncthreads();
+      if (wave > 0) return;
+      uint32_t base = 0;  // items (11 bits), slots (11 bits), splits (10 bits) so far
+      for (int t0 = 0; t0 < tiles; t0 += 64) {
+        const uint2 tile = s_list[t0 + lane < tiles ? t0 + lane : 0];
+        const int steps = int(tile.y);
+        int n = steps > s_most ? ceil_div(steps, s_most) : 1;
+        n = t0 + lane < tiles ? n : 0;
+        const uint32_t mine = uint32_t(n) | (n > 1 ? (uint32_t(n) << 11) | (1u << 22) : 0u);
+        uint32_t incl = mine;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const uint32_t y = __shfl_up(incl, off);
+          incl += lane >= off ? y : 0u;
+        }
+        const uint32_t at = base + incl - mine;
+        uint32_t word = uint32_t(n) << 10;
+        if (n > 1) {
+          word |= ((at >> 11) & 2047u) << 20;
+          const int seq = int(tile.x >> 12), row0 = int(tile.x & 0xfffu) * QT, q0 = p.cu[seq];
+          const int rows = p.cu[seq + 1] - q0 - row0;
+          p.splits[at >> 22] = make_uint4(q0 + row0, rows < QT ? rows : QT, word, 0);
+        }
+        for (int k = 0; k < n; ++k) {
+          const int i = int(at & 2047u) + k;
+          if (i < p.max_items) p.items[i] = make_uint2(tile.x, word | uint32_t(k));
+        }
+        base += __shfl(incl, 63);
+      }
+      if (lane == 0) {
+        const int items = int(base & 2047u);
+        p.n_items[0] = items < p.max_items ? items : p.max_items;
+        p.n_items[1] = int(base >> 22);
+      }
+      return;
+    }
+  }
+  for (int b = tid; b < kBuckets; b += 1024) bucket[b] = 0;
+  // Bucket of query tile qt: the key tokens it visits, most work first.
+  auto bucket_of = [&](int reach) { return nbk - 1 - reach / 256; };
+  for_each_tile([&](int, int, int reach) { atomicAdd(&bucket[bucket_of(reach)], 1); });
   __syncthreads();
   {
     static_assert(kBuckets <= 64 * 17, "bucket_prefix covers 17 buckets per lane");
     const int run = bucket_prefix<17>(bucket, nbk - 1, 0, tid);
-    if (tid == 0) *p.n_items = run < p.max_items ? run : p.max_items;
+    if (tid == 0) {
+      p.n_items[0] = run < p.max_items ? run : p.max_items;
+      p.n_items[1] = 0;
+    }
   }
-  for_each_tile([&](int seq, int qt, int b) {
-    const int slot = atomicAdd(&bucket[b], 1);
-    if (slot < p.max_items) p.items[slot] = (uint32_t(seq) << 12) | uint32_t(qt);
+  for_each_tile([&](int seq, int qt, int reach) {
+    const int at = atomicAdd(&bucket[bucket_of(reach)], 1);
+    if (at < p.max_items) p.items[at] = make_uint2((uint32_t(seq) << 12) | uint32_t(qt), 1u << 10);
   });
 }
 
@@ -189,7 +294,8 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void varlen_prefill_kernel(Pref
   const int it = int(blockIdx.x) / p.kv_heads;
   const int kvh = int(blockIdx.x) - it * p.kv_heads;
   if (it >= *p.n_items) return;
-  const uint32_t e = p.items[it];
+  const uint2 item = p.items[it];
+  const uint32_t e = uint32_t(uniform(int(item.x))), word = uint32_t(uniform(int(item.y)));
   const int seq = int(e >> 12), qt = int(e & 0xfffu);
   const int tid = threadIdx.x, lane = tid & 63, w = uniform(int(tid >> 6));
   const int c = lane & 15, g = lane >> 4;
@@ -241,13 +347,19 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void varlen_prefill_kernel(Pref
   // wave for a memory round trip per tile. The window moves (one vector load)
   // when a tile leaves it.
   const int n_blocks = range_end > 0 ? (range_end - 1) / p.block_size + 1 : 0;
-  int win0 = 0;
-  int lane_blk = lane < n_blocks ? table_row[lane] : 0;
+  // Steps [first_step, first_step + n_steps) of the tile: all, or this piece's.
+  const int n_parts = pieces_of(word);
+  const int all_steps = ((range_end + kPrefillTile - 1) / kPrefillTile + KT - 1) / KT;
+  const int part_steps = (all_steps + n_parts - 1) / n_parts;
+  const int first_step = piece_of(word) * part_steps;
+  const int n_steps = all_steps - first_step < part_steps ? all_steps - first_step : part_steps;
+  int win0 = first_step * KT * kPrefillTile / p.block_size;
+  int lane_blk = win0 + lane < n_blocks ? table_row[win0 + lane] : 0;
   const uint32_t ring_base = lds_addr(ring);
-  // Tile ti goes to ring slot ti % (S * KT). Tiles past the range (the second
+  // Tile ti of the piece goes to ring slot ti % (S * KT). Tiles past the range (the second
   // tile of a last, half-used step) move no bytes and land as zeros.
   auto issue = [&](int ti) {
-    const int t0 = ti * kPrefillTile;
+    const int t0 = (first_step * KT + ti) * kPrefillTile;
     if (t0 >= range_end) {
       const u32x4 rz = raw_rsrc(p.k_cache, 0u);
       const uint32_t slot = ring_base + uint32_t(ti % (S * KT)) * RG::SLOT;
@@ -415,12 +527,13 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void varlen_prefill_kernel(Pref
   // immediate offsets instead of per-step address arithmetic).
   static_assert(S >= 2, "one step resident, one in flight");
   constexpr int PER_STEP = KT * RG::NIW;  // direct-to-LDS loads per wave per step
-  const int n_tiles = (range_end + kPrefillTile - 1) / kPrefillTile;
-  const int n_steps = (n_tiles + KT - 1) / KT;
   auto issue_step = [&](int si) {
 #pragma unroll
     for (int h = 0; h < KT; ++h) issue(si * KT + h);
   };
+  // The block ids and q are complete here by a wait the compiler accounts for:
+  // without it, it drains the tile loads in flight on every tile (see `issue`).
+  __builtin_amdgcn_s_waitcnt(kVmcntZero);
   if (n_steps > 0) {
 #pragma unroll
     for (int i = 0; i < S - 1; ++i)
@@ -438,12 +551,25 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void varlen_prefill_kernel(Pref
           __syncthreads();
           if (si + S - 1 < n_steps) issue_step(si + S - 1);
           qk(ring + u * STEP, sc);
-          finish(ring + u * STEP, si * KT * kPrefillTile, sc);
+          finish(ring + u * STEP, (first_step + si) * KT * kPrefillTile, sc);
         }
       }
     }
   }
 
+  if (n_parts > 1) {
+    const int64_t base = (int64_t(slot_of(word) + piece_of(word)) * p.kv_heads + kvh) * (QT * G);
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if (!live[nb]) continue;
+      const int64_t col = base + (w * NB + nb) * 16 + c;
+      float *po = p.part_o + col * D + 4 * g;
+#pragma unroll
+      for (int b = 0; b < VPL; ++b) *reinterpret_cast<f32x4 *>(po + 16 * b) = oacc[nb][b];
+      if (g == 0) p.part_ml[col] = make_float2(m_run[nb], lacc[nb][0]);
+    }
+    return;
+  }
 #pragma unroll
   for (int nb = 0; nb < NB; ++nb) {
     const float l_tot = lacc[nb][0];
@@ -460,10 +586,72 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void varlen_prefill_kernel(Pref
   }
 }
 
+// Combine the pieces of the tiles that were cut: one wave per (tile, kv head,
+// column), lane l owning D / 64 dims, four pieces' loads in flight at a time. A
+// fixed grid walks all columns, so calls whose tiles stayed whole pay only an
+// empty launch.
+constexpr int kMergeThreads = 512;
+template <int D>
+__global__ __launch_bounds__(kMergeThreads) void prefill_merge_kernel(PrefillParams p, int cols) {
+  constexpr int V = D / 64, W = kMergeThreads / 64;
+  const int lane = threadIdx.x & 63;
+  const int per_tile = p.kv_heads * cols;
+  const int total = ld_const(p.n_items + 1) * per_tile;
+  for (int i = uniform(int(blockIdx.x * W + (threadIdx.x >> 6))); i < total; i += int(gridDim.x) * W) {
+    const int t = i / per_tile, kvh = (i - t * per_tile) / cols, col = i - t * per_tile - kvh * cols;
+    const uint32_t *split = &p.splits[t].x;
+    const uint32_t word = ld_const(split + 2);
+    const int q0 = int(ld_const(split)), n = pieces_of(word), row = col / p.group;
+    if (row >= int(ld_const(split + 1))) continue;
+    const int64_t base = (int64_t(slot_of(word)) * p.kv_heads + kvh) * cols + col;
+    const int64_t stride = int64_t(p.kv_heads) * cols;
+    float m_run = -INFINITY, l = 0.0f, acc[V];
+#pragma unroll
+    for (int v = 0; v < V; ++v) acc[v] = 0.0f;
+    for (int k0 = 0; k0 < n; k0 += 4) {
+      float m[4], pl[4], o[4][V];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int64_t r = base + (k0 + j < n ? k0 + j : n - 1) * stride;
+        m[j] = ld_const(&p.part_ml[r].x);
+        pl[j] = ld_const(&p.part_ml[r].y);
+        const float *po = p.part_o + r * D + V * lane;
+#pragma unroll
+        for (int v = 0; v < V; ++v) o[j][v] = po[v];
+      }
+#pragma unroll
+      for (int j = 1; j < 4; ++j) m[j] = k0 + j < n ? m[j] : -INFINITY;
+      const float m_new = fmaxf(fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3])), m_run);
+      if (m_new == -INFINITY) continue;  // no key of these pieces is visible
+      const float alpha = fast_exp2(m_run - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int v = 0; v < V; ++v) acc[v] *= alpha;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float f = fast_exp2(m[j] - m_new);
+        l += f * pl[j];
+#pragma unroll
+        for (int v = 0; v < V; ++v) acc[v] += k0 + j < n ? f * o[j][v] : 0.0f;
+      }
+      m_run = m_new;
+    }
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    uint16_t *op = p.out + ((int64_t(q0) + row) * p.q_heads + kvh * p.group + col % p.group) * D + V * lane;
+    if constexpr (V == 1) {
+      op[0] = uint16_t(f32_to_bf16_bits(acc[0] * inv));
+    } else {
+#pragma unroll
+      for (int v = 0; v < V; v += 2)
+        *reinterpret_cast<uint32_t *>(op + v) = pack_bf16x2(acc[v] * inv, acc[v + 1] * inv);
+    }
+  }
+}
+
 namespace {
 
 template <int D>
-void launch_prefill(const PrefillParams &p, int grid, hipStream_t s) {
+void launch_prefill(const PrefillParams &p, int grid, int merge_grid, hipStream_t s) {
   const dim3 g(grid * p.kv_heads);
   switch (p.group) {
     case 1: varlen_prefill_kernel<D, 1><<<g, 64 * kPrefillWaves, 0, s>>>(p); break;
@@ -472,10 +660,23 @@ void launch_prefill(const PrefillParams &p, int grid, hipStream_t s) {
     case 8: varlen_prefill_kernel<D, 8><<<g, 64 * kPrefillWaves, 0, s>>>(p); break;
     default: varlen_prefill_kernel<D, 16><<<g, 64 * kPrefillWaves, 0, s>>>(p); break;
   }
+  if (merge_grid > 0)
+    prefill_merge_kernel<D><<<merge_grid, kMergeThreads, 0, s>>>(p, prefill_q_tile(D, p.group) * p.group);
 }
 
-uint64_t prefill_items_bound(int num_seqs, int total_q, int q_tile) {
+uint64_t prefill_tiles_bound(int num_seqs, int total_q, int q_tile) {
   return uint64_t(total_q) / q_tile + uint64_t(num_seqs) + 1;
+}
+// Bytes of the work list, for the smallest query tile (head_dim 256, group 16) and
+// the pieces that cutting may add.
+uint64_t prefill_items_bytes(int num_seqs, int total_q) {
+  return 16 + align16(8 * (prefill_tiles_bound(num_seqs, total_q, prefill_q_tile(256, 16)) +
+                           uint64_t(device_cus())));
+}
+uint64_t prefill_splits_bytes() { return sizeof(uint4) * uint64_t(device_cus()); }
+// Partial columns: at most one (piece, kv head) pair per CU.
+uint64_t prefill_partial_columns(int head_dim) {
+  return uint64_t(device_cus()) * (kPrefillWaves * prefill_nb(head_dim) * 16);
 }
 
 }  // namespace
@@ -488,7 +689,8 @@ extern "C" uint64_t ifattn_varlen_prefill_workspace_size(int32_t num_seqs, int32
                                                          int32_t max_kv_len) {
   if (num_seqs <= 0 || total_q <= 0 || q_heads <= 0 || head_dim <= 0 || max_kv_len <= 0) return 0;
   const uint64_t dec = split_k_workspace_bytes(num_seqs, q_heads, head_dim, max_kv_len);
-  return align16(dec) + 16 + 4 * prefill_items_bound(num_seqs, total_q, 1);
+  return align16(dec) + prefill_items_bytes(num_seqs, total_q) + prefill_splits_bytes() +
+         prefill_partial_columns(head_dim) * (4 * uint64_t(head_dim) + sizeof(float2));
 }
 
 extern "C" int32_t ifattn_varlen_prefill_bf16(const void *q, const void *k_cache, const void *v_cache,
@@ -558,8 +760,14 @@ extern "C" int32_t ifattn_varlen_prefill_bf16(const void *q, const void *k_cache
     uint8_t *w = static_cast<uint8_t *>(workspace) +
                  align16(split_k_workspace_bytes(num_seqs, q_heads, head_dim, max_kv_len));
     p.n_items = reinterpret_cast<int32_t *>(w);
-    p.items = reinterpret_cast<uint32_t *>(w + 16);
+    p.items = reinterpret_cast<uint2 *>(w + 16);
+    w += prefill_items_bytes(num_seqs, total_q);
+    p.splits = reinterpret_cast<uint4 *>(w);
+    w += prefill_splits_bytes();
+    p.part_ml = reinterpret_cast<float2 *>(w);
+    p.part_o = reinterpret_cast<float *>(p.part_ml + prefill_partial_columns(head_dim));
   }
+  p.cus = device_cus();
   p.num_blocks = num_blocks;
   p.num_seqs = num_seqs;
   p.q_heads = q_heads;
@@ -573,13 +781,20 @@ extern "C" int32_t ifattn_varlen_prefill_bf16(const void *q, const void *k_cache
   if (int64_t(max_q_len) > int64_t(4096) * p.q_tile)
     return fail(IFATTN_EINVAL, "varlen prefill: max_q_len above 4096 query tiles per sequence");
   p.max_q_len = max_q_len;
-  const int grid = int(prefill_items_bound(num_seqs, total_q, p.q_tile));
+  // Enough query tiles for one per CU even if every other sequence is a decode row:
+  // no tile is cut. The plan gets the same answer, as the device's cu_seqlens may
+  // hold fewer rows than total_q.
+  const bool may_split = (int64_t(total_q) - num_seqs) / p.q_tile * kv_heads < p.cus &&
+                         max_kv_len > kMinPieceKeys + kMinSavedKeys;
+  const int grid = int(prefill_tiles_bound(num_seqs, total_q, p.q_tile)) +
+                   (may_split ? p.cus / kv_heads : 0);
   p.max_items = grid;
 
   launch_varlen_decode_rows(d, head_dim, s);
-  prefill_plan_kernel<<<1, 1024, 0, s>>>(p);
-  if (head_dim == 64) launch_prefill<64>(p, grid, s);
-  else if (head_dim == 128) launch_prefill<128>(p, grid, s);
-  else launch_prefill<256>(p, grid, s);
+  prefill_plan_kernel<<<1, 1024, 0, s>>>(p, prefill_kt(head_dim) * kPrefillTile, may_split);
+  const int merge_grid = may_split ? 4 * p.cus : 0;
+  if (head_dim == 64) launch_prefill<64>(p, grid, merge_grid, s);
+  else if (head_dim == 128) launch_prefill<128>(p, grid, merge_grid, s);
+  else launch_prefill<256>(p, grid, merge_grid, s);
   return launch_status("varlen prefill");
 }
