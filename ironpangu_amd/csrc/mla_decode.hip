@@ -82,7 +82,7 @@ struct MlaParams {
                                 // writes its output directly
   int32_t *start_row;           // [max_workers] first row not wholly before each worker's share
   uint16_t *part_o;             // [slots, heads, 512] scaled fp16 O / l of each partial
-  float *part_ml;               // [slots, heads, 8] m, l, two unused, inverse scale of each 128 dims
+  f32x4 *part_ml;               // [slots, heads, 4] m, l, inverse scale of 128 dims, unused
   int64_t num_blocks;
   uint32_t cache_bytes;  // sparse and row-quantized gathers: byte extent of the cache (< 4 GiB - 16)
   uint32_t scale_bytes;  // row-quantized rows: byte extent of row_scales
@@ -507,12 +507,13 @@ constexpr uint32_t kNoRow = 0xFFFFFFFFu;  // sparse slot list: no key
 // precision (error against 64 bits of a window-2048 call 0.0026 with bf16
 // partials, 0.0021). Stores a lane's 32 consecutive dims (o times inv), scaled
 // over the four lanes (g) that share the wave's 128, to partial row prow, and
-// the wave's entry of its (m, l, scales).
+// the wave's (m, l, inverse scale), which the merge reads as one 16-byte load.
 __device__ __forceinline__ void mla_store_partial(const MlaParams &p, int64_t prow, int w, int g,
                                                   const float (&o)[32], float inv, float m, float l) {
-  float amax = 0.0f;
+  float mx[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // four chains: no other work hides their latency
 #pragma unroll
-  for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(o[i]));
+  for (int i = 0; i < 32; ++i) mx[i & 3] = fmaxf(mx[i & 3], fabsf(o[i]));
+  const float amax = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
   const float ps = f16_range_scale(max_xor32(max_xor16(amax * inv)));
   const float f = inv * ps;
   uint16_t *po = p.part_o + prow * 512 + 128 * w + 32 * g;
@@ -522,11 +523,8 @@ __device__ __forceinline__ void mla_store_partial(const MlaParams &p, int64_t pr
   };
 #pragma unroll
   for (int k = 0; k < 32; k += 8) store_u32x4(po + k, u32x4{two(k), two(k + 2), two(k + 4), two(k + 6)});
-  if (g == 0) {
-    float *e = p.part_ml + prow * 8;
-    e[4 + w] = __uint_as_float((254u << 23) - __float_as_uint(ps));  // 1 / ps
-    if (w == 0) *reinterpret_cast<float2 *>(e) = make_float2(m, l);
-  }
+  if (g == 0)
+    p.part_ml[prow * 4 + w] = f32x4{m, l, __uint_as_float((254u << 23) - __float_as_uint(ps)), 0.0f};
 }
 
 __device__ __forceinline__ int mla_tile_token(int g, int j) {
@@ -1652,7 +1650,9 @@ __global__ __launch_bounds__(64 * (MlaCfg<F, false, WIDE>::NW), (MlaCfg<F, false
 // Combine one (row, head): the row's partials (the sink partial first, when
 // there are sinks, then one per share its tiles touch). Bound by round trips,
 // not bytes, so all of them are loaded at once. Up to kFast partials: every
-// thread loads its two dims and (m, l) of each. More: wave u takes partials u,
+// thread loads its two dims and (m, l, scale) of each (16 bytes in one vector load; as
+// three scalar loads, with the partials past the last repeated, a window call
+// of 128 rows took 70.6 us instead of 69.8). More: wave u takes partials u,
 // u + 4, ... (lane l dims 8l .. 8l + 7, up to kBatch 16-byte loads in flight, those
 // past the last partial out of the buffer's range), every wave reads all (m, l)
 // (lane k: partial k) and takes the weights from them, and the waves' sums meet in
@@ -1663,26 +1663,32 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
   constexpr int kBatch = 8, kFast = 8;
   const int row = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int wv = uniform(tid >> 6);
+  // All arguments in one round trip (the compiler would load the later ones behind
+  // the row's slots).
+  asm volatile("" ::"s"(p.row_slot), "s"(p.part_ml), "s"(p.part_o), "s"(p.out), "s"(p.heads));
   const int2 slots = make_int2(ld_const(&p.row_slot[row].x), ld_const(&p.row_slot[row].y));
   if (slots.x < 0) return;  // output written by the attention kernel or the plan
   const int total = slots.y;
   const int64_t prow0 = int64_t(slots.x) * p.heads + h;
   uint32_t *op = reinterpret_cast<uint32_t *>(p.out + (int64_t(row) * p.heads + h) * 512) + tid;
   if (total <= kFast) {
-    float2 ml[kFast];
-    float sc[kFast];
+    f32x4 ml[kFast];
     uint32_t o[kFast];
 #pragma unroll
-    for (int k = 0; k < kFast; ++k) {  // indices past the last partial repeat it with weight 0
-      const int64_t r = prow0 + int64_t(k < total ? k : total - 1) * p.heads;
-      const float *e = p.part_ml + r * 8;  // wave-uniform: scalar loads
-      ml[k] = make_float2(ld_const(e), ld_const(e + 1));
-      sc[k] = ld_const(e + 4 + wv);
-      o[k] = *reinterpret_cast<const uint32_t *>(p.part_o + r * 512 + 2 * tid);
+    for (int k = 0; k < kFast; ++k) {
+      ml[k] = f32x4{-INFINITY, 0.0f, 0.0f, 0.0f};
+      o[k] = 0u;
+      if (k < total) {
+        const int64_t r = prow0 + int64_t(k) * p.heads;
+        // A vector load: eight 16-byte scalar ones wait for each other's registers.
+        ml[k] = *reinterpret_cast<const f32x4 *>(
+            reinterpret_cast<const char *>(p.part_ml + r * 4) + 16u * (uint32_t(tid) >> 6));
+        o[k] = *reinterpret_cast<const uint32_t *>(p.part_o + r * 512 + 2 * tid);
+      }
     }
     float mx = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < kFast; ++k) mx = fmaxf(mx, ml[k].x);
+    for (int k = 0; k < kFast; ++k) mx = fmaxf(mx, ml[k][0]);
     if (mx == -INFINITY) {  // nothing visible
       *op = 0u;
       return;
@@ -1690,10 +1696,10 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
     float l = 0.0f, o0 = 0.0f, o1 = 0.0f;
 #pragma unroll
     for (int k = 0; k < kFast; ++k) {  // partials hold O / l
-      const float wk = k < total ? fast_exp2(ml[k].x - mx) * ml[k].y : 0.0f;
+      const float wk = fast_exp2(ml[k][0] - mx) * ml[k][1];
       const f16x2 x = pair(o[k]);
       l += wk;
-      const float f = wk * sc[k];
+      const float f = wk * ml[k][2];
       o0 += f * float(x[0]);
       o1 += f * float(x[1]);
     }
@@ -1704,7 +1710,7 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
   __shared__ float s_acc[4][512];
   const uint32_t stride = uint32_t(p.heads), rows = uint32_t(total) * stride;
   const auto ro = make_rsrc(p.part_o + prow0 * 512, rows * 1024u);
-  const auto rm = make_rsrc(p.part_ml + prow0 * 8, rows * 32u);
+  const auto rm = make_rsrc(p.part_ml + prow0 * 4, rows * 64u);
   u32x4 o[kBatch];
   float sc[kBatch];
   auto load = [&](int k0) {
@@ -1712,13 +1718,13 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(MlaParams p) {
     for (int u = 0; u < kBatch; ++u) {
       const uint32_t r = uint32_t(k0 + wv + 4 * u) * stride;
       o[u] = buf_load_x4(ro, r * 1024u + 16u * uint32_t(lane));
-      sc[u] = buf_load_f32(rm, r * 32u + 16u + 4u * uint32_t(lane >> 4));
+      sc[u] = buf_load_f32(rm, r * 64u + 8u + 16u * uint32_t(lane >> 4));
     }
   };
   load(0);
   // (m, l) of partial k + lane, and the largest m of all partials.
   auto load_ml = [&](int k) {
-    const uint32_t off = uint32_t(k + lane) * stride * 32u;
+    const uint32_t off = uint32_t(k + lane) * stride * 64u;
     return make_float2(k + lane < total ? buf_load_f32(rm, off) : -INFINITY, buf_load_f32(rm, off + 4));
   };
   float2 ml = load_ml(0);
@@ -1895,7 +1901,7 @@ inline uint64_t mla_workspace(int rows, int heads, bool sparse, int topk, int n_
   const uint64_t workers = mla_max_workers(sparse, rows, topk, n_sinks);
   const uint64_t slots = mla_slots(workers, rows, n_sinks);
   return kQueueBytes + 2 * align16(uint64_t(rows) * 8) + align16(uint64_t(rows) * 4) +
-         align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 8 * sizeof(float));
+         align16(workers * 4) + slots * heads * (512 * sizeof(uint16_t) + 4 * sizeof(f32x4));
 }
 
 int32_t mla_run(const MlaCall &c, const char *what) {
@@ -1999,7 +2005,7 @@ int32_t mla_run(const MlaCall &c, const char *what) {
   ws += align16(max_workers * 4);
   const uint64_t slots = mla_slots(max_workers, c.num_rows, c.n_sinks);
   p.part_o = reinterpret_cast<uint16_t *>(ws);
-  p.part_ml = reinterpret_cast<float *>(p.part_o + slots * c.heads * 512);
+  p.part_ml = reinterpret_cast<f32x4 *>(p.part_o + slots * c.heads * 512);
   hipStream_t s = static_cast<hipStream_t>(c.stream);
   if (!p.self_plan) mla_plan_kernel<<<1, 1024, 0, s>>>(p);
   constexpr int kThreads = 64 * kMlaWaves;
