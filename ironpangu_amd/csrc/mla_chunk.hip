@@ -13,7 +13,7 @@
 // from L2; it takes 2.2-2.4 us (2.2 without the loads). A group's start (q and
 // the first tile) takes 6 us and its partial output 6 us. Measured against the
 // row-by-row kernel: 756 rows x 16 heads in three chunks, window 2048, 128
-// sinks 269 -> 105 us a call with the writer; 2048 rows over 8192 earlier keys
+// sinks 267 -> 91 us a call with the writer; 2048 rows over 8192 earlier keys
 // 688 us (954 TFLOP/s).
 //
 // Layout: eight waves, two per SIMD. Scores are split by columns: wave w owns

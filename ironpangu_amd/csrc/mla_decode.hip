@@ -1025,8 +1025,9 @@ __device__ __forceinline__ void mla_item(const MlaParams &p, uint8_t *ring, floa
 // Bound: VALU, 694 instructions per wave and 64 keys (about 360 dequantize the
 // wave's keys, 192 convert V), each SIMD's VALU busy 69% of the time; the row
 // loads alone take 0.2 ms of the int8 call below. int8 rows, 128 sequences of
-// 1024..65536 keys: 0.363 -> 0.262 ms (0.277 with unrotated rows, whose score
-// reads kept the LDS in bank conflicts half the time); int4 rows 0.345 -> 0.303 ms.
+// 1024..65536 keys: 0.363 -> 0.248 ms with the merge of many partials (0.262 with
+// the former one, then 0.277 with unrotated rows, whose score reads kept the LDS in
+// bank conflicts half the time); int4 rows 0.345 -> 0.303 ms.
 // Eight waves with 128-key steps in one workgroup per CU ran 0.321 ms: the
 // phases of a step then wait for each other with nothing beside them.
 template <int F>
