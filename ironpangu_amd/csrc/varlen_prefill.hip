@@ -86,13 +86,13 @@ __device__ __forceinline__ int ceil_div(int a, int b) {
 // kMinSavedKeys (about 12 us at 3 us per 128 keys, against 9 us for partials and
 // merge), and into pieces of at least kMinPieceKeys (a piece's start costs as
 // much as two steps).
-constexpr int kMinPieceKeys = 256, kMinSavedKeys = 512;
+constexpr int kMinPieceKeys = 256, kMinSavedKeys = 512, kMinIdleKeys = 400;
 constexpr int kMaxCutTiles = 1024;
 
 // Work list for the multi-row sequences. Enough items for every CU: sorted by the
 // number of key tokens the query tile visits (descending, 256-token buckets).
 // Fewer (tile, kv head) items than CUs (and the caller launches the merge:
-// may_split): their order does not matter, and the tiles are cut into pieces of
+// MAY_SPLIT): their order does not matter, and the tiles are cut into pieces of
 // at most `most` steps, the smallest of 16 candidates with which the items still
 // fit one per CU (pieces of the average load make more items than CUs: a second
 // round, 77 us for the prompts below). Bound otherwise by the longest item's walk.
@@ -101,12 +101,12 @@ constexpr int kMaxCutTiles = 1024;
 // chunks at head_dim 256 130 -> 76, at 64 with 8 kv heads 183 -> 64.
 // The cut path keeps to wave scans: LDS atomics with per-lane values run lane by
 // lane (8.5 us for the plan instead of 4.3).
-__global__ __launch_bounds__(1024) void prefill_plan_kernel(PrefillParams p, int step_keys,
-                                                            bool may_split) {
+template <bool MAY_SPLIT>
+__global__ __launch_bounds__(1024) void prefill_plan_kernel(PrefillParams p, int step_keys) {
   constexpr int kBuckets = 1025;
   __shared__ int bucket[kBuckets];
   __shared__ int s_count[1024], s_kv[1024];
-  __shared__ uint2 s_list[kMaxCutTiles];  // (seq << 12 | tile, steps)
+  __shared__ uint2 s_list[MAY_SPLIT ? kMaxCutTiles : 1];  // (seq << 12 | tile, steps)
   __shared__ int s_tiles, s_most;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int QT = p.q_tile;
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(1024) void prefill_plan_kernel(PrefillParams p, int
       }
     }
   };
-  if (may_split) {
+  if constexpr (MAY_SPLIT) {
     for_each_tile([&](int seq, int qt, int reach) {
       const int at = atomicAdd(&s_tiles, 1);
       if (at < kMaxCutTiles)
@@ -358,10 +358,10 @@ __global__ __launch_bounds__(64 * kPrefillWaves) void varlen_prefill_kernel(Pref
   // Steps [first_step, first_step + n_steps) of the tile: all, or this piece's.
   const int n_parts = pieces_of(word);
   const int all_steps = ((range_end + kPrefillTile - 1) / kPrefillTile + KT - 1) / KT;
-  const int part_steps = (all_steps + n_parts - 1) / n_parts;
+  const int part_steps = uniform(ceil_div(all_steps, n_parts));
   const int first_step = piece_of(word) * part_steps;
   const int n_steps = all_steps - first_step < part_steps ? all_steps - first_step : part_steps;
-  int win0 = first_step * KT * kPrefillTile / p.block_size;
+  int win0 = first_step * KT * kPrefillTile >> __builtin_ctz(p.block_size);  // a power of two
   int lane_blk = win0 + lane < n_blocks ? table_row[win0 + lane] : 0;
   const uint32_t ring_base = lds_addr(ring);
   // Tile ti of the piece goes to ring slot ti % (S * KT). Tiles past the range (the second
@@ -789,17 +789,26 @@ extern "C" int32_t ifattn_varlen_prefill_bf16(const void *q, const void *k_cache
   if (int64_t(max_q_len) > int64_t(4096) * p.q_tile)
     return fail(IFATTN_EINVAL, "varlen prefill: max_q_len above 4096 query tiles per sequence");
   p.max_q_len = max_q_len;
-  // Enough query tiles for one per CU even if every other sequence is a decode row:
-  // no tile is cut. The plan gets the same answer, as the device's cu_seqlens may
-  // hold fewer rows than total_q.
-  const bool may_split = (int64_t(total_q) - num_seqs) / p.q_tile * kv_heads < p.cus &&
-                         max_kv_len > kMinPieceKeys + kMinSavedKeys;
+  // The least number of query tiles, every other sequence taken as a decode row. No
+  // tile is cut if they make an item per CU; and cutting is only tried (it costs
+  // the merge launch and a longer plan, 3 us) where the longest walk times the
+  // share of idle CUs is kMinIdleKeys: three prompts of 187..1777 rows, 470 keys,
+  // 62.4 -> 54.1 us a call; eight chunks of 197..590 rows over up to 847 keys, 340,
+  // stay whole and would take 59.3 us instead of 56.8. The plan gets the same
+  // answer, as the device's cu_seqlens may hold fewer rows than total_q.
+  const int64_t items = (int64_t(total_q) - num_seqs) / p.q_tile * kv_heads;
+  const bool may_split = items < p.cus && max_kv_len > kMinPieceKeys + kMinSavedKeys &&
+                         max_kv_len * (p.cus - items) >= int64_t(kMinIdleKeys) * p.cus;
   const int grid = int(prefill_tiles_bound(num_seqs, total_q, p.q_tile)) +
                    (may_split ? p.cus / kv_heads : 0);
   p.max_items = grid;
 
   launch_varlen_decode_rows(d, head_dim, s);
-  prefill_plan_kernel<<<1, 1024, 0, s>>>(p, prefill_kt(head_dim) * kPrefillTile, may_split);
+  const int step_keys = prefill_kt(head_dim) * kPrefillTile;
+  if (may_split)
+    prefill_plan_kernel<true><<<1, 1024, 0, s>>>(p, step_keys);
+  else
+    prefill_plan_kernel<false><<<1, 1024, 0, s>>>(p, step_keys);
   const int merge_grid = may_split ? 4 * p.cus : 0;
   if (head_dim == 64) launch_prefill<64>(p, grid, merge_grid, s);
   else if (head_dim == 128) launch_prefill<128>(p, grid, merge_grid, s);
